@@ -785,6 +785,373 @@ __global__ __launch_bounds__(kFThreads, 1) void fp8_gemm_256_kernel(GemmParams p
   }
 }
 
+// ---------------------------------------------------------------- smaller tiles for small outputs
+//
+// The same GEMM on tiles of 32 WN TN (n) x 32 WM TM (m), WN x WM waves of 32 TN x 32 TM each, for
+// outputs whose 256 x 256 / 256 x 128 tiles would leave most compute units idle. A stage holds the
+// tile's W rows then its X rows, 128 K bytes each, in the same swizzle (row block offsets are
+// multiples of 32, which leave it unchanged), in a ring of NST stages with NST - 1 in flight: one
+// barrier a stage publishes stage s and retires every wave's reads of stage s - 1, whose buffer the
+// loads issued right after it refill. Every output is one chain of 32x32x64 MFMAs over K in order,
+// as in the 256-row tiles, so the result does not depend on the tile chosen.
+template <int BN, int BM>
+constexpr int ring_stage_bytes() { return (BN + BM) * kFBK; }
+
+// f(R), f(R - 1), ..., f(0) with compile-time arguments.
+template <int R, typename F>
+__device__ __forceinline__ void unrolled_down(F f) {
+  f(std::integral_constant<int, R>{});
+  if constexpr (R > 0) unrolled_down<R - 1>(f);
+}
+
+// The scaled bf16 epilogue of a BN x BM tile staged through LDS (row r: BN * 2 bytes, 16-byte chunk
+// c at c ^ (r % (BN / 8))), with the options of staged_epilogue: residual, per-group maxima, and
+// (XD > 0) the q / k transform read head-major. Lane owns m = 32 (TM wm + j) + lane % 32 and
+// n = 32 (TN wn + i) + 8 g + 4 (lane / 32) + 0..3.
+template <int WN, int WM, int TN, int TM, int XD>
+__device__ __forceinline__ void ring_epilogue(const GemmParams& p, const v16f (&acc)[TN][TM], uint8_t* lds, int m0,
+                                              int n0, int wave, int lane, int split) {
+  constexpr int BN = 32 * WN * TN, BM = 32 * WM * TM, NW = WN * WM;
+  constexpr int CPR = BN / 8;                     // 16-byte chunks of a row
+  constexpr int ROWB = BN * 2;
+  const int wn = wave % WN, wm = wave / WN, hh = lane >> 5, tid = wave * 64 + lane;
+  if (p.part) {                                   // split-K: unscaled fp32 partials, 16-byte stores
+    float* base = p.part + (int64_t)split * p.M * p.N;
+#pragma unroll
+    for (int i = 0; i < TN; ++i)
+#pragma unroll
+      for (int j = 0; j < TM; ++j) {
+        const int m = m0 + 32 * (TM * wm + j) + (lane & 31);
+#pragma unroll
+        for (int g = 0; g < 4; ++g) {
+          const int n = n0 + 32 * (TN * wn + i) + 8 * g + 4 * hh;
+          const v16f& c = acc[i][j];
+          if (m < p.M && n < p.N)
+            *reinterpret_cast<float4*>(base + (int64_t)m * p.N + n) =
+                make_float4(c[4 * g], c[4 * g + 1], c[4 * g + 2], c[4 * g + 3]);
+        }
+      }
+    return;
+  }
+#pragma unroll
+  for (int i = 0; i < TN; ++i) {
+    float swn[16];
+#pragma unroll
+    for (int g = 0; g < 4; ++g) {
+      const int n = min(n0 + 32 * (TN * wn + i) + 8 * g + 4 * hh, p.N - 4);
+      if (p.sw_step) {
+        const float4 v = *reinterpret_cast<const float4*>(p.sw + n);
+        swn[4 * g] = v.x; swn[4 * g + 1] = v.y; swn[4 * g + 2] = v.z; swn[4 * g + 3] = v.w;
+      } else {
+#pragma unroll
+        for (int e = 0; e < 4; ++e) swn[4 * g + e] = p.sw[0];
+      }
+    }
+#pragma unroll
+    for (int j = 0; j < TM; ++j) {
+      const int r = 32 * (TM * wm + j) + (lane & 31), m = m0 + r;
+      const float sxm = p.sx[(int64_t)min(m, p.M - 1) * p.sx_step];
+      const v16f& c = acc[i][j];
+#pragma unroll
+      for (int g = 0; g < 4; ++g) {
+        float v[4];
+#pragma unroll
+        for (int e = 0; e < 4; ++e) v[e] = c[4 * g + e] * sxm * swn[4 * g + e];
+        if (!p.lds_epi) {                         // rows that 16-byte stores cannot take
+          const int n = n0 + 32 * (TN * wn + i) + 8 * g + 4 * hh;
+          if (m < p.M && n < p.N) {               // N % 4 == 0
+            if (p.res) {
+              const uint2 rr = *reinterpret_cast<const uint2*>(p.res + (int64_t)m * p.rs + n);
+              v[0] = round_bf16(v[0]) + __uint_as_float(rr.x << 16);
+              v[1] = round_bf16(v[1]) + __uint_as_float(rr.x & 0xFFFF0000u);
+              v[2] = round_bf16(v[2]) + __uint_as_float(rr.y << 16);
+              v[3] = round_bf16(v[3]) + __uint_as_float(rr.y & 0xFFFF0000u);
+            }
+            *reinterpret_cast<uint2*>(p.y + (int64_t)m * p.ys + n) =
+                make_uint2(pack_bf16x2(v[0], v[1]), pack_bf16x2(v[2], v[3]));
+          }
+        } else {
+          const int ch = 4 * (TN * wn + i) + g;
+          *reinterpret_cast<uint2*>(lds + r * ROWB + 16 * (ch ^ (r & (CPR - 1))) + 8 * hh) =
+              make_uint2(pack_bf16x2(v[0], v[1]), pack_bf16x2(v[2], v[3]));
+        }
+      }
+    }
+  }
+  if (!p.lds_epi) return;
+  __builtin_amdgcn_s_waitcnt(0xC07F);             // lgkmcnt(0)
+  lds_barrier();
+  auto staged_at = [&](int r, int ch) __attribute__((always_inline)) {
+    return *reinterpret_cast<const uint4*>(lds + r * ROWB + 16 * (ch ^ (r & (CPR - 1))));
+  };
+  auto store_at = [&](int r, int ch, uint4 o, flw_u16x2& mx) __attribute__((always_inline)) {
+    const int m = m0 + r, n = n0 + 8 * ch;
+    if (m < p.M && n < p.N) {
+      if (p.res) {
+        const uint4 rr = *reinterpret_cast<const uint4*>(p.res + (int64_t)m * p.rs + n);
+        const uint32_t a[4] = {o.x, o.y, o.z, o.w}, b[4] = {rr.x, rr.y, rr.z, rr.w};
+        uint32_t ov[4];
+#pragma unroll
+        for (int e = 0; e < 4; ++e)
+          ov[e] = pack_bf16x2(__uint_as_float(a[e] << 16) + __uint_as_float(b[e] << 16),
+                              __uint_as_float(a[e] & 0xFFFF0000u) + __uint_as_float(b[e] & 0xFFFF0000u));
+        o = make_uint4(ov[0], ov[1], ov[2], ov[3]);
+      }
+      *reinterpret_cast<uint4*>(p.y + (int64_t)m * p.ys + n) = o;
+      if (p.gmax) {
+        mx = abs_max_bf16x2(mx, o.x);
+        mx = abs_max_bf16x2(mx, o.y);
+        mx = abs_max_bf16x2(mx, o.z);
+        mx = abs_max_bf16x2(mx, o.w);
+      }
+    }
+  };
+  // Group maxima of the waves, past the staged tile.
+  uint32_t* red = reinterpret_cast<uint32_t*>(lds + BM * ROWB);
+  const int lpg = p.gmax ? min(p.gcols >> 3, CPR) : 1;      // chunks of a column group in the tile
+  if constexpr (XD > 0) {
+    // Head-major: LPR lanes per head row, each the same 8 columns of every head of the tile.
+    constexpr int LPR = XD / 8, RPP = 64 / LPR, HPT = BN / XD, RPW = BM / NW, NB = RPW / RPP;
+    static_assert(BN % XD == 0 && RPW % RPP == 0, "a wave's rows are whole batches");
+    const int xsub = lane / LPR, xdc = lane % LPR;
+    const bool xform = n0 < p.xcols, rope = xform && p.rcos != nullptr;     // uniform
+    flw_u16x2 lmh[HPT];
+#pragma unroll
+    for (int h = 0; h < HPT; ++h) lmh[h] = flw_u16x2{0, 0};
+    auto batch = [&](auto hw, int r, const uint4 (&v)[HPT], const float* cf, const float* sf)
+        __attribute__((always_inline)) {
+#pragma unroll
+      for (int h = 0; h < HPT; ++h) {
+        const int nh = n0 + h * XD;               // uniform
+        if (nh >= p.N) break;
+        uint4 o = v[h];
+        if (nh < p.xcols) {
+          float f[8];
+          Vec16<uint16_t>::unpack(o, f);
+          uint32_t pk[4] = {o.x, o.y, o.z, o.w};
+          head_norm_rope_core<uint16_t, decltype(hw)::value>(f, p.xnorm != 0, p.xeps, XD, LPR, true, rope, cf, sf,
+                                                             pk);
+          o = make_uint4(pk[0], pk[1], pk[2], pk[3]);
+        }
+        store_at(r, h * LPR + xdc, o, lmh[h]);
+      }
+    };
+#pragma unroll 1
+    for (int b = 0; b < NB; ++b) {
+      const int r = RPW * wave + RPP * b + xsub;
+      uint4 tc = make_uint4(0, 0, 0, 0), tsn = tc;
+      if (rope) {                                 // rows past M use the last row's entries
+        const int64_t off = (int64_t)((uint32_t)min(m0 + r, p.M - 1) % (uint32_t)p.xT) * XD + 8 * xdc;
+        tc = *reinterpret_cast<const uint4*>(p.rcos + off);
+        tsn = *reinterpret_cast<const uint4*>(p.rsin + off);
+      }
+      uint4 v[HPT];
+      flw_u16x2 fm = {0, 0};                      // max |x| of the values transformed
+#pragma unroll
+      for (int h = 0; h < HPT; ++h) {
+        v[h] = staged_at(r, h * LPR + xdc);
+        if (n0 + h * XD < min(p.N, p.xcols)) {
+          fm = abs_max_bf16x2(fm, v[h].x);
+          fm = abs_max_bf16x2(fm, v[h].y);
+          fm = abs_max_bf16x2(fm, v[h].z);
+          fm = abs_max_bf16x2(fm, v[h].w);
+        }
+      }
+      float cf[8], sf[8];
+      Vec16<uint16_t>::unpack(tc, cf);
+      Vec16<uint16_t>::unpack(tsn, sf);
+      // The pair converter only where no NaN can arise: every input finite, eps > 0.
+      const bool bad = (fm[0] > fm[1] ? fm[0] : fm[1]) >= 0x7F80u || (p.xnorm != 0 && !(p.xeps > 0.0f));
+      if (__builtin_amdgcn_ballot_w64(bad) == 0) batch(std::true_type{}, r, v, cf, sf);
+      else batch(std::false_type{}, r, v, cf, sf);
+    }
+    // Every lane of a wave holds rows of every head: the wave's max per head.
+#pragma unroll
+    for (int h = 0; h < HPT; ++h) {
+      const uint32_t v = wave_max_u32(lmh[h][0] > lmh[h][1] ? lmh[h][0] : lmh[h][1]);
+      if (lane == 0) red[wave * CPR + h] = v;
+    }
+  } else {
+    flw_u16x2 lm = {0, 0};                        // max |y| bf16 bits of this lane's chunk column
+    static_assert((64 * NW) % CPR == 0, "a thread keeps its chunk column");
+    const int ch = tid % CPR;
+#pragma unroll 4
+    for (int q = 0; q < BM * CPR / (64 * NW); ++q) {
+      const int r = (q * 64 * NW + tid) / CPR;
+      store_at(r, ch, staged_at(r, ch), lm);
+    }
+    if (p.gmax) {
+      // Lanes of one column group, then the lanes that hold other rows of the same columns.
+      uint32_t v = lm[0] > lm[1] ? lm[0] : lm[1];
+#pragma unroll
+      for (int o = 1; o < 64; o <<= 1) {
+        const uint32_t t = (uint32_t)__shfl_xor((int)v, o, 64);
+        if (o < lpg || o >= CPR) v = v > t ? v : t;
+      }
+      if (lane < CPR && (ch & (lpg - 1)) == 0) red[wave * CPR + ch / lpg] = v;
+    }
+  }
+  if (p.gmax) {
+    // One atomic max per group and tile (gcols may exceed the tile's width: then per tile column).
+    __builtin_amdgcn_s_waitcnt(0xC07F);
+    lds_barrier();
+    if (tid < CPR / lpg && n0 + 8 * lpg * tid < p.N) {
+      uint32_t mx = 0;
+#pragma unroll
+      for (int w = 0; w < NW; ++w) mx = mx > red[w * CPR + tid] ? mx : red[w * CPR + tid];
+      atomicMax(p.gmax + (n0 + 8 * lpg * tid) / p.gcols, mx << 16);     // bf16 bits -> fp32 bits
+    }
+  }
+  // The next tile's loads refill the ring: every wave's reads of the staged tile are done.
+  __builtin_amdgcn_s_waitcnt(0xC07F);
+  lds_barrier();
+}
+
+template <int WN, int WM, int TN, int TM, int NST, int XD = 0, bool HALFK = false, bool PIPE = false>
+__global__ __launch_bounds__(64 * WN * WM) void fp8_gemm_ring_kernel(GemmParams p) {
+  constexpr int BN = 32 * WN * TN, BM = 32 * WM * TM, NW = WN * WM;
+  constexpr int kStage = ring_stage_bytes<BN, BM>();
+  constexpr int IPW = (BN + BM) / 8 / NW;         // loads of 8 rows per wave and stage
+  static_assert((BN + BM) % (8 * NW) == 0 && IPW * (NST - 1) < 64, "whole instructions, countable by vmcnt");
+  static_assert(NST * kStage >= BM * BN * 2 + NW * BN / 2, "the staged epilogue and its maxima reuse the ring");
+  __shared__ __align__(16) uint8_t lds[NST * kStage];
+  const int tid = threadIdx.x, lane = tid & 63;
+  const int wave = __builtin_amdgcn_readfirstlane(tid >> 6);
+  const int wn = wave % WN, wm = wave / WN;
+  const uint32_t lds0 = (uint32_t)(uintptr_t)(lds_u8_t*)lds;
+  const uint8_t *const w8 = p.w8, *const x8 = p.x8;
+  const int nst_all = (p.K + kFBK - 1) / kFBK;    // the last one 64 deep when K % 128 == 64
+  const int G = gridDim.x;
+  const int L = (G & 7) == 0 ? (blockIdx.x & 7) * (G >> 3) + (blockIdx.x >> 3) : blockIdx.x;
+  const int ntiles = p.tiles_n * p.tiles_m;
+  for (int item = L; item < ntiles * p.splits; item += G) {
+    const int split = item / ntiles, t = item % ntiles;
+    const int group = t / (kGroupM * p.tiles_n);
+    const int first_m = group * kGroupM;
+    const int gm = min(p.tiles_m - first_m, kGroupM);
+    const int m0 = (first_m + (t % (kGroupM * p.tiles_n)) % gm) * BM;
+    const int n0 = ((t % (kGroupM * p.tiles_n)) / gm) * BN;
+    // Split-K: this item's K stages.
+    const int sbase = split * nst_all / p.splits, nst = (split + 1) * nst_all / p.splits - sbase;
+    const bool half_last = HALFK && sbase + nst == nst_all;
+    // Lane i of instruction q fetches row 8 q + i / 8 of the wave's rows, LDS position i % 8, i.e.
+    // global chunk (i % 8) ^ swizzle; rows past M / N fetch the last valid row (not stored).
+    uint32_t goff[IPW];
+    uint32_t hi_half = 0;                         // bit q: instruction q's chunk is in bytes 64-127
+#pragma unroll
+    for (int q = 0; q < IPW; ++q) {
+      const int row0 = 8 * (wave * IPW + q);
+      const bool xop = row0 >= BN;
+      const int r = (xop ? row0 - BN : row0) + (lane >> 3);
+      const int c = (lane & 7) ^ ((r >> 1) & 7);
+      const int grow = xop ? min(m0 + r, p.M - 1) : min(n0 + r, p.N - 1);
+      goff[q] = (uint32_t)grow * (uint32_t)p.K + 16u * (uint32_t)c;
+      hi_half |= (uint32_t)(c >> 2) << q;
+    }
+    auto issue = [&](int s) __attribute__((always_inline)) {
+      const uint32_t dst = lds0 + (uint32_t)(s % NST) * kStage;
+      const uint32_t back = half_last && s == nst - 1 ? 64u : 0u;   // the last stage's bytes 64-127: 0-63 again
+#pragma unroll
+      for (int q = 0; q < IPW; ++q) {
+        const int row0 = 8 * (wave * IPW + q);
+        const uint8_t* src = row0 >= BN ? x8 : w8;
+        asm volatile("s_mov_b32 m0, %0\n\tglobal_load_lds_dwordx4 %1, %2"
+                     :: "s"(dst + row0 * 128), "v"(goff[q] + (uint32_t)(sbase + s) * kFBK - (((hi_half >> q) & 1u) ? back : 0u)),
+                        "s"(src) : "memory", "m0");
+      }
+    };
+    v16f acc[TN][TM];
+#pragma unroll
+    for (int i = 0; i < TN; ++i)
+#pragma unroll
+      for (int j = 0; j < TM; ++j) acc[i][j] = v16f{};
+#pragma unroll
+    for (int s = 0; s < NST - 1; ++s)
+      if (s < nst) issue(s);
+    v8i a[2][2][TN], b[2][2][TM];                 // fragments [parity][K chunk][block]
+    auto read = [&](int s, auto pc) __attribute__((always_inline)) {
+      constexpr int P = decltype(pc)::value;
+      const uint8_t* cur = lds + (s % NST) * kStage;
+#pragma unroll
+      for (int kc = 0; kc < 2; ++kc) {
+#pragma unroll
+        for (int i = 0; i < TN; ++i) a[P][kc][i] = swz_frag(cur, TN * wn + i, kc, lane);
+#pragma unroll
+        for (int j = 0; j < TM; ++j) b[P][kc][j] = swz_frag(cur, BN / 32 + TM * wm + j, kc, lane);
+      }
+    };
+    auto prod = [&](auto pc, auto kcc) __attribute__((always_inline)) {
+      constexpr int P = decltype(pc)::value, kc = decltype(kcc)::value;
+#pragma unroll
+      for (int i = 0; i < TN; ++i)
+#pragma unroll
+        for (int j = 0; j < TM; ++j) acc[i][j] = gemm_mfma(a[P][kc][i], b[P][kc][j], acc[i][j]);
+    };
+    using C0 = std::integral_constant<int, 0>;
+    using C1 = std::integral_constant<int, 1>;
+    auto mult = [&](int s, bool last) __attribute__((always_inline)) {
+      read(s, C0{});
+      prod(C0{}, C0{});
+      if (!(half_last && last)) prod(C0{}, C1{});
+      __builtin_amdgcn_s_waitcnt(0xC07F);         // lgkmcnt(0): this wave's reads of stage s are done
+    };
+    auto fetch = [&](int s, auto pc) __attribute__((always_inline)) {
+      __builtin_amdgcn_s_waitcnt(vmcnt_imm((NST - 2) * IPW));   // this wave's loads of stage s landed
+      lds_barrier();                              // ... and every wave's; stage s - 1 is retired
+      issue(s + NST - 1);
+      read(s, pc);
+    };
+    if constexpr (PIPE) {
+      if (nst >= NST) {
+        int s = 0;
+        fetch(0, C0{});
+#pragma unroll 1
+        for (; s + NST + 1 < nst; s += 2) {
+          __builtin_amdgcn_s_waitcnt(0xC07F);
+          prod(C0{}, C0{});
+          fetch(s + 1, C1{});
+          prod(C0{}, C1{});
+          __builtin_amdgcn_s_waitcnt(0xC07F);
+          prod(C1{}, C0{});
+          fetch(s + 2, C0{});
+          prod(C1{}, C1{});
+        }
+        __builtin_amdgcn_s_waitcnt(0xC07F);
+        prod(C0{}, C0{});
+        if (s + NST < nst) {
+          fetch(s + 1, C1{});
+          prod(C0{}, C1{});
+          __builtin_amdgcn_s_waitcnt(0xC07F);
+          prod(C1{}, C0{});
+          prod(C1{}, C1{});
+        } else {
+          prod(C0{}, C1{});
+        }
+      }
+    } else {
+#pragma unroll 1
+      for (int s = 0; s + NST - 1 < nst; ++s) {
+        __builtin_amdgcn_s_waitcnt(vmcnt_imm((NST - 2) * IPW));   // this wave's loads of stage s landed
+        lds_barrier();                              // ... and every wave's; stage s - 1 is retired
+        issue(s + NST - 1);
+        mult(s, false);
+      }
+    }
+    // The last NST - 1 stages: nothing left to issue, r stages still in flight behind each.
+    auto tail = [&](auto rc) __attribute__((always_inline)) {
+      constexpr int r = decltype(rc)::value;
+      if (r < nst) {
+        __builtin_amdgcn_s_waitcnt(vmcnt_imm(r * IPW));
+        lds_barrier();
+        mult(nst - 1 - r, r == 0);
+      }
+    };
+    unrolled_down<NST - 2>(tail);
+    lds_barrier();                                // the epilogue overwrites the ring
+    ring_epilogue<WN, WM, TN, TM, XD>(p, acc, lds, m0, n0, wave, lane, split);
+  }
+}
+
 // Split-K finish: y[m, n..n+3] = bf16( (sum_s part[s][m][n]) * sx[m] * sw[n] ) (+ residual as in
 // the one-pass epilogue); one thread per 4 outputs.
 __global__ __launch_bounds__(256) void gemm_splitk_reduce_kernel(GemmParams p) {
@@ -1022,10 +1389,9 @@ __global__ __launch_bounds__(256) void fill_u32_kernel(uint32_t* p, int n, uint3
 
 // Compute units of the current device (queried once per device).
 
-// K ranges per output tile for the 256 x 256 kernel: split when the tiles alone would leave more
-// than half of the compute units idle and each range keeps at least 4 K stages of 128. (Measured
-// at the C2 shapes: the wgrad output [4096, 1024], 64 tiles, 96 -> 54 us with 4 ranges; the dgrad
-// output [8192, 1024], 128 tiles, gains nothing from 2.)
+// K ranges per output tile a caller's workspace is sized for (flw_fp8_scaled_mm_workspace_bytes):
+// outputs whose 256 x 256 tiles would leave more than half of the compute units idle, each range
+// keeping at least 4 K stages of 128. Whether the GEMM then splits is use_split's decision.
 static int splitk_of(int64_t tiles, int64_t K) {
   const int cus = compute_units();
   if (tiles * 2 >= cus) return 1;     // half the GPU or more busy: the finish pass would cost more
@@ -1040,6 +1406,75 @@ static size_t splitk_bytes(int64_t M, int64_t N, int64_t K) {
   const int64_t tiles = ((N + kFBN - 1) / kFBN) * ((M + kFBM - 1) / kFBM);
   const int sp = splitk_of(tiles, K);
   return sp > 1 ? (size_t)sp * (size_t)M * (size_t)N * sizeof(float) : 0;
+}
+
+// Split over K only where 256 x 256 tiles x 3 ranges fill the GPU and K is long enough to pay for
+// the partials: [3840, 1280] and [3392, 1280] at K = 16384 93 / 90 us against 102 / 99 us unsplit,
+// 61 / 59 against 53 / 52 us at K = 8192. Every other split measured slower than the smaller tiles
+// unsplit: [4096, 1024] at K = 8192 48 -> 37 us, [1024, 1024] at K = 4096 24 -> 10 us.
+static bool use_split(int splits, int64_t K) { return splits == 3 && K >= 96 * kFBK; }
+
+// Output tiles of the FP8 GEMM, n x m. Every one accumulates an output's K products in the same
+// order, so the choice changes the time only.
+enum class Tile { k64x32, k64x64, k128x64, k128x128, k128x128Pair, k256x128, k256x256 };
+
+// The tile for an [M, N] output (K % 64 == 0). While one of the smaller tiles gives at most one tile
+// per compute unit, the largest such: a tile's time hardly depends on how many others run (K =
+// 4096, us: 8.5 / 9 / 10.5 / 15 / 28 / 48 for 64x32 / 64x64 / 128x64 / 128x128 / 256x128 / 256x256),
+// so a small output takes the smallest that fits in one round ([16, 1024] at K = 4096 28 -> 8.2 us,
+// [2048, 1024] 30 -> 13.4 us, [1024, 3072] at K = 1024 11.0 -> 8.0 us). Up to two 128 x 128 tiles
+// per unit and K >= 2048, two workgroups share a unit ([4096, 1280] at K = 3392: 32 -> 29 us, the
+// same at K = 1024). Beyond that the rounds of the persistent grid decide between the two large
+// tiles, a round of 256 x 128 tiles taking 0.55 of one of 256 x 256 ([4096, 3392] at K = 1280:
+// 29.0 -> 26.0 us on 224 wide tiles; [8192, 1280] at K = 3392, 160 wide tiles: 62 -> 52 us).
+// Figures with operands that alternate among buffers larger than the L2s.
+static Tile tile_of(int64_t M, int64_t N, int64_t K, bool narrow_ok) {
+  const int64_t cus = compute_units();
+  auto count = [M, N](int64_t bn, int64_t bm) { return ((N + bn - 1) / bn) * ((M + bm - 1) / bm); };
+  if (count(64, 32) <= cus) return Tile::k64x32;
+  if (count(64, 64) <= cus) return Tile::k64x64;
+  if (count(128, 64) <= cus) return Tile::k128x64;
+  const int64_t pairs = count(128, 128);
+  if (pairs <= cus) return Tile::k128x128;
+  if (pairs <= 2 * cus && (K >= 2048 || !narrow_ok)) return Tile::k128x128Pair;
+  const double wide = (double)((count(256, 256) + cus - 1) / cus);
+  const double narrow = 0.55 * (double)((count(256, 128) + cus - 1) / cus);
+  return narrow_ok && narrow < wide ? Tile::k256x128 : Tile::k256x256;
+}
+
+struct TileKernel {
+  const void* fn;
+  int bn, bm, threads, per_cu;        // per_cu: workgroups that fit a compute unit's LDS
+};
+
+// XD: head dim of the q / k transform epilogue (0: none; HALFK never set with it).
+template <int XD, bool HALFK>
+static TileKernel tile_kernel(Tile t) {
+  switch (t) {
+    case Tile::k64x32:
+      if constexpr (XD == 0)
+        return {reinterpret_cast<const void*>(&fp8_gemm_ring_kernel<2, 1, 1, 1, 4, 0, HALFK>), 64, 32, 128, 3};
+      [[fallthrough]];
+    case Tile::k64x64:
+      if constexpr (XD == 0)
+        return {reinterpret_cast<const void*>(&fp8_gemm_ring_kernel<2, 2, 1, 1, 4, 0, HALFK, true>), 64, 64, 256, 2};
+      [[fallthrough]];
+    case Tile::k128x64:
+      if constexpr (XD == 0)
+        return {reinterpret_cast<const void*>(&fp8_gemm_ring_kernel<4, 2, 1, 1, 4, 0, HALFK, true>), 128, 64, 512, 1};
+      else    // 16 rows a wave, whole row batches of the head-major epilogue
+        return {reinterpret_cast<const void*>(&fp8_gemm_ring_kernel<2, 2, 2, 1, 3, XD, HALFK, true>), 128, 64, 256, 2};
+    case Tile::k128x128:
+      return {reinterpret_cast<const void*>(&fp8_gemm_ring_kernel<4, 2, 1, 2, 3, XD, HALFK, true>), 128, 128, 512, 1};
+    case Tile::k128x128Pair:
+      return {reinterpret_cast<const void*>(&fp8_gemm_ring_kernel<4, 2, 1, 2, 2, XD, HALFK>), 128, 128, 512, 2};
+    case Tile::k256x128:
+      if constexpr (XD == 0)
+        return {reinterpret_cast<const void*>(&fp8_gemm_256_kernel<128, 0, HALFK>), 256, 128, kFThreads, 1};
+      [[fallthrough]];
+    default:
+      return {reinterpret_cast<const void*>(&fp8_gemm_256_kernel<256, XD, HALFK>), 256, 256, kFThreads, 1};
+  }
 }
 
 static int scaled_mm(const uint8_t* x8, int64_t M, int64_t K, const uint8_t* w8, int64_t N,
@@ -1065,51 +1500,34 @@ static int scaled_mm(const uint8_t* x8, int64_t M, int64_t K, const uint8_t* w8,
   FLW_REQUIRE(res == nullptr || (rs >= N && rs % 4 == 0 && ((uintptr_t)res & 7) == 0), FLW_E_INVALID,
               "residual rows must be 8-byte aligned with a stride >= N, a multiple of 4");
   if (K % 64 == 0 && N * K < (1ll << 32) && M * K < (1ll << 32)) {
-    p.tiles_n = (int)((N + kFBN - 1) / kFBN);
-    p.tiles_m = (int)((M + kFBM - 1) / kFBM);
-    const int64_t tiles = (int64_t)p.tiles_n * p.tiles_m;
-    FLW_REQUIRE(tiles <= 0x7FFFFFFF, FLW_E_UNSUPPORTED, "grid too large");
-    // Split-K into the caller's workspace when the output has too few tiles to fill the GPU.
+    const int64_t wide = ((N + kFBN - 1) / kFBN) * ((M + kFBM - 1) / kFBM);
+    FLW_REQUIRE(wide <= 0x7FFFFFFF, FLW_E_UNSUPPORTED, "grid too large");
     p.splits = 1;
     p.lds_epi = N % 8 == 0 && ys % 8 == 0 && ((uintptr_t)y & 15) == 0 &&
                 (res == nullptr || (rs % 8 == 0 && ((uintptr_t)res & 15) == 0));
-    const size_t need = splitk_bytes(M, N, K);
-    if (need && workspace && workspace_bytes >= need && ((uintptr_t)workspace & 15) == 0 && N % 4 == 0) {
-      p.splits = splitk_of(tiles, K);
+    // Split-K into the caller's workspace.
+    const int splits = splitk_of(wide, K);
+    // 256 x 128 tiles have the staged epilogue only, and no group maxima in it.
+    Tile tile = tile_of(M, N, K, p.lds_epi != 0 && gmax == nullptr);
+    if (use_split(splits, K) && workspace && workspace_bytes >= splitk_bytes(M, N, K) &&
+        ((uintptr_t)workspace & 15) == 0) {
+      p.splits = splits;
       p.part = static_cast<float*>(workspace);
-    }
-    // Fewer 256 x 256 tiles than compute units: 256 x 128 tiles (twice as many), and then half
-    // the K ranges of an even split (the same number of work items, half the partials to fold).
-    // An odd split keeps its 256 x 256 tiles: halving 3 ranges to 1 would leave the items a
-    // third of the GPU short (the 450M block's wgrad outputs [3392 | 3840, 1280] at K = 16384:
-    // 70 / 75 tiles x 3 ranges, 97 / 92 us against 108 / 103 us as 135 / 150 narrow tiles).
-    // More tiles than compute units: the narrow tiles too when they fill the last round of the
-    // persistent grid enough better to pay their ~10 % higher cost per output (measured at
-    // M = 16384: 320 tiles [N = 1280] 62.5 % -> 83 % filled, -10 to -19 %; 896 tiles 87.5 % ->
-    // 100 %, -3 %; 960 or 512 tiles, equally filled either way, +3 to +13 % narrow).
-    const int cus = compute_units();
-    auto fill = [cus](int64_t items) { return (double)items / (double)(((items + cus - 1) / cus) * cus); };
-    const bool narrow = p.lds_epi && gmax == nullptr && xform == nullptr &&
-                        (tiles < cus ? (p.splits == 1 || p.splits % 2 == 0)
-                                     : p.splits == 1 && fill(2 * tiles) > 1.1 * fill(tiles));
-    if (narrow) {
-      p.tiles_m = (int)((M + 127) / 128);
-      p.splits = p.splits / 2 > 1 ? p.splits / 2 : 1;
-      if (p.splits == 1) p.part = nullptr;
+      tile = Tile::k256x256;
     }
     // K % 128 == 64 (no q / k transform: its entry point requires K % 128 == 0): the instances
     // whose last K stage is 64 deep.
-    const bool halfk = K % kFBK != 0;
-    const void* kern = narrow ? (halfk ? reinterpret_cast<const void*>(&fp8_gemm_256_kernel<128, 0, true>)
-                                       : reinterpret_cast<const void*>(&fp8_gemm_256_kernel<128>))
-                     : xform == nullptr ? (halfk ? reinterpret_cast<const void*>(&fp8_gemm_256_kernel<256, 0, true>)
-                                                 : reinterpret_cast<const void*>(&fp8_gemm_256_kernel<256>))
-                     : gcols == 32 ? reinterpret_cast<const void*>(&fp8_gemm_256_kernel<256, 32>)
-                     : gcols == 64 ? reinterpret_cast<const void*>(&fp8_gemm_256_kernel<256, 64>)
-                     : reinterpret_cast<const void*>(&fp8_gemm_256_kernel<256, 128>);
-    // Persistent: one workgroup per CU (each holds 128 KB of LDS), at most one per work item.
-    const int64_t items = (int64_t)p.tiles_n * p.tiles_m * p.splits;
-    const int64_t grid = items < compute_units() ? items : compute_units();
+    const TileKernel k = xform == nullptr ? (K % kFBK != 0 ? tile_kernel<0, true>(tile) : tile_kernel<0, false>(tile))
+                         : gcols == 32    ? tile_kernel<32, false>(tile)
+                         : gcols == 64    ? tile_kernel<64, false>(tile)
+                                          : tile_kernel<128, false>(tile);
+    const int64_t tiles_n = (N + k.bn - 1) / k.bn, tiles_m = (M + k.bm - 1) / k.bm;
+    p.tiles_n = (int)tiles_n;
+    p.tiles_m = (int)tiles_m;
+    // Persistent: as many workgroups as the compute units hold at once, at most one per work item.
+    const int64_t items = tiles_n * tiles_m * p.splits, slots = (int64_t)compute_units() * k.per_cu;
+    FLW_REQUIRE(items <= 0x7FFFFFFF - slots, FLW_E_UNSUPPORTED, "grid too large");
+    const dim3 grid((unsigned)(items < slots ? items : slots)), block((unsigned)k.threads);
     if (gmax) {
       FLW_REQUIRE(p.splits == 1 && p.lds_epi, FLW_E_UNSUPPORTED,
                   "the group amax needs an unsplit GEMM with N %% 8 == 0 and 16-byte aligned rows");
@@ -1123,13 +1541,12 @@ static int scaled_mm(const uint8_t* x8, int64_t M, int64_t K, const uint8_t* w8,
       const int ng = (int)(N / gcols);
       (void)launch_args(reinterpret_cast<const void*>(&fill_u32_kernel), dim3((unsigned)((ng + 255) / 256)),
                         dim3(256), 0, s, tm.start, nullptr, gmax, ng, 0u);
-      (void)launch_ext(kern, dim3((unsigned)grid), dim3(kFThreads), 0, s, p, nullptr, tm.stop);
+      (void)launch_ext(k.fn, grid, block, 0, s, p, nullptr, tm.stop);
     } else if (p.splits == 1) {
-      (void)launch_timed(kern, dim3((unsigned)grid), dim3(kFThreads), s, p);
+      (void)launch_timed(k.fn, grid, block, s, p);
     } else {
       const Timer tm = take_timer();
-      (void)launch_ext(kern, dim3((unsigned)grid), dim3(kFThreads),
-                       0, s, p, tm.start, nullptr);
+      (void)launch_ext(k.fn, grid, block, 0, s, p, tm.start, nullptr);
       const int64_t quads = M * (N / 4);
       (void)launch_ext(reinterpret_cast<const void*>(&gemm_splitk_reduce_kernel), dim3((unsigned)((quads + 255) / 256)),
                        dim3(256), 0, s, p, nullptr, tm.stop);
