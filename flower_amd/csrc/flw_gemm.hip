@@ -33,7 +33,7 @@ constexpr int kCPT = kChunks / 256;              // 4 per thread
 struct GemmParams {
   const uint8_t* x8;   // [M, K]
   const uint8_t* w8;   // [N, K]
-  const float* sx;     // M or 1
+  const float* sx;     // M or 1 (ring_epilogue: null is 1.0)
   const float* sw;     // N or 1
   int sx_step, sw_step;
   uint16_t* y;         // [M, N] bf16
@@ -850,7 +850,7 @@ __device__ __forceinline__ void ring_epilogue(const GemmParams& p, const v16f (&
 #pragma unroll
     for (int j = 0; j < TM; ++j) {
       const int r = 32 * (TM * wm + j) + (lane & 31), m = m0 + r;
-      const float sxm = p.sx[(int64_t)min(m, p.M - 1) * p.sx_step];
+      const float sxm = p.sx ? p.sx[(int64_t)min(m, p.M - 1) * p.sx_step] : 1.0f;
       const v16f& c = acc[i][j];
 #pragma unroll
       for (int g = 0; g < 4; ++g) {
@@ -1382,6 +1382,114 @@ __global__ __launch_bounds__(kFThreads, 1) void w8a16_gemm_kernel(W8A16Params p)
   }
 }
 
+// The same product on the ring kernel's smaller tiles (fp8_gemm_ring_kernel: tiles, ring, epilogue),
+// for outputs with too few 256 x 256 tiles; a stage is 64 deep, the tile's X rows (128 bytes, as
+// above) then its W rows (64 bytes). An output's products accumulate in w8a16_tile's order.
+template <int WN, int WM, int TN, int TM, int NST>
+__global__ __launch_bounds__(64 * WN * WM) void w8a16_ring_kernel(W8A16Params p) {
+  constexpr int BN = 32 * WN * TN, BM = 32 * WM * TM, NW = WN * WM;
+  constexpr int kXIns = BM / 8, kStage = BM * 128 + BN * 64;
+  constexpr int IPW = (kXIns + BN / 16) / NW;     // loads (8 X rows or 16 W rows) per wave and stage
+  static_assert((kXIns + BN / 16) % NW == 0 && IPW * (NST - 1) < 64, "whole instructions, countable by vmcnt");
+  static_assert(NST * kStage >= BM * BN * 2 + NW * BN / 2, "the staged epilogue reuses the ring");
+  __shared__ __align__(16) uint8_t lds[NST * kStage];
+  const int tid = threadIdx.x, lane = tid & 63;
+  const int wave = __builtin_amdgcn_readfirstlane(tid >> 6);
+  const int wn = wave % WN, wm = wave / WN, h = lane >> 5;
+  const uint32_t lds0 = (uint32_t)(uintptr_t)(lds_u8_t*)lds;
+  const uint16_t* const x = p.x;
+  const uint8_t* const w8 = p.w8;
+  GemmParams e{};                                 // the epilogue's part
+  e.sw = p.sw; e.sw_step = p.sw_step; e.y = p.y; e.ys = p.ys; e.M = p.M; e.N = p.N; e.lds_epi = p.lds_epi;
+  const int nst = p.K / kWK;
+  const int G = gridDim.x;
+  const int L = (G & 7) == 0 ? (blockIdx.x & 7) * (G >> 3) + (blockIdx.x >> 3) : blockIdx.x;
+  const int ntiles = p.tiles_n * p.tiles_m;
+  for (int t = L; t < ntiles; t += G) {
+    const int group = t / (kGroupM * p.tiles_n);
+    const int first_m = group * kGroupM;
+    const int gm = min(p.tiles_m - first_m, kGroupM);
+    const int m0 = (first_m + (t % (kGroupM * p.tiles_n)) % gm) * BM;
+    const int n0 = ((t % (kGroupM * p.tiles_n)) / gm) * BN;
+    uint32_t off[IPW];                            // rows past M / N fetch the last valid row
+#pragma unroll
+    for (int q = 0; q < IPW; ++q) {
+      const int ins = wave * IPW + q;
+      if (ins < kXIns) {
+        const int r = 8 * ins + (lane >> 3), c = (lane & 7) ^ ((r >> 1) & 7);
+        off[q] = (uint32_t)min(m0 + r, p.M - 1) * (uint32_t)(p.xs * 2) + 16u * (uint32_t)c;
+      } else {
+        const int r = 16 * (ins - kXIns) + (lane >> 2), c = (lane & 3) ^ ((r >> 2) & 3);
+        off[q] = (uint32_t)min(n0 + r, p.N - 1) * (uint32_t)p.K + 16u * (uint32_t)c;
+      }
+    }
+    auto issue = [&](int s) __attribute__((always_inline)) {
+      const uint32_t dst = lds0 + (uint32_t)(s % NST) * kStage;
+#pragma unroll
+      for (int q = 0; q < IPW; ++q) {
+        const int ins = wave * IPW + q;
+        if (ins < kXIns)
+          asm volatile("s_mov_b32 m0, %0\n\tglobal_load_lds_dwordx4 %1, %2"
+                       :: "s"(dst + ins * 1024), "v"(off[q] + (uint32_t)s * (kWK * 2)), "s"(x) : "memory", "m0");
+        else
+          asm volatile("s_mov_b32 m0, %0\n\tglobal_load_lds_dwordx4 %1, %2"
+                       :: "s"(dst + ins * 1024), "v"(off[q] + (uint32_t)s * kWK), "s"(w8) : "memory", "m0");
+      }
+    };
+    v16f acc[TN][TM];
+#pragma unroll
+    for (int i = 0; i < TN; ++i)
+#pragma unroll
+      for (int j = 0; j < TM; ++j) acc[i][j] = v16f{};
+#pragma unroll
+    for (int s = 0; s < NST - 1; ++s)
+      if (s < nst) issue(s);
+    auto mult = [&](int s) __attribute__((always_inline)) {
+      const uint8_t* cur = lds + (s % NST) * kStage;
+      v8bf_t b[TM][4];
+#pragma unroll
+      for (int j = 0; j < TM; ++j) {
+        const int r = 32 * (TM * wm + j) + (lane & 31);
+#pragma unroll
+        for (int ks = 0; ks < 4; ++ks)
+          b[j][ks] = bf16_frag(*reinterpret_cast<const uint4*>(cur + swz_off(r, 4 * h + ks)));
+      }
+      const uint8_t* wt = cur + BM * 128;
+#pragma unroll
+      for (int i = 0; i < TN; ++i) {
+        const int r = 32 * (TN * wn + i) + (lane & 31);
+        const uint4 q0 = *reinterpret_cast<const uint4*>(wt + wswz_off(r, 2 * h));
+        const uint4 q1 = *reinterpret_cast<const uint4*>(wt + wswz_off(r, 2 * h + 1));
+        const v8bf_t a[4] = {widen8(q0.x, q0.y), widen8(q0.z, q0.w), widen8(q1.x, q1.y), widen8(q1.z, q1.w)};
+#pragma unroll
+        for (int ks = 0; ks < 4; ++ks)
+#pragma unroll
+          for (int j = 0; j < TM; ++j)
+            acc[i][j] = __builtin_amdgcn_mfma_f32_32x32x16_bf16(a[ks], b[j][ks], acc[i][j], 0, 0, 0);
+      }
+      __builtin_amdgcn_s_waitcnt(0xC07F);         // lgkmcnt(0): this wave's reads of stage s are done
+    };
+#pragma unroll 1
+    for (int s = 0; s + NST - 1 < nst; ++s) {
+      __builtin_amdgcn_s_waitcnt(vmcnt_imm((NST - 2) * IPW));   // this wave's loads of stage s landed
+      lds_barrier();                              // ... and every wave's; stage s - 1 is retired
+      issue(s + NST - 1);
+      mult(s);
+    }
+    auto tail = [&](auto rc) __attribute__((always_inline)) {   // r stages still in flight behind it
+      constexpr int r = decltype(rc)::value;
+      if (r < nst) {
+        __builtin_amdgcn_s_waitcnt(vmcnt_imm(r * IPW));
+        lds_barrier();
+        mult(nst - 1 - r);
+      }
+    };
+    unrolled_down<NST - 2>(tail);
+    lds_barrier();                                // the epilogue overwrites the ring
+    ring_epilogue<WN, WM, TN, TM, 0>(e, acc, lds, m0, n0, wave, lane, 0);
+  }
+}
+
 __global__ __launch_bounds__(256) void fill_u32_kernel(uint32_t* p, int n, uint32_t v) {
   const int i = blockIdx.x * 256 + threadIdx.x;
   if (i < n) p[i] = v;
@@ -1563,6 +1671,25 @@ static int scaled_mm(const uint8_t* x8, int64_t M, int64_t K, const uint8_t* w8,
   return check_launch("flw_fp8_scaled_mm");
 }
 
+// The W8A16 product's tile: while 64 x 64 or 128 x 64 (n x m) give at most one tile per compute unit,
+// the first of them ([200, 3840] at K = 1280 30.6 -> 8.6 us, [512, 1024] at K = 4096 83 -> 20, [2048,
+// 1024] at K = 4096 85 -> 25); beyond that 128 x 128 tiles, two workgroups a unit, or 256 x 256, by
+// the rounds: in units of a 256 x 256 round a full one of the pairs takes 0.64, a last one of at most
+// a tile per unit 0.39 ([4096, 1024] at K = 1024 26 -> 13 us, [8192, 3072] 63 -> 55; [8192, 4096] stays
+// on 256 x 256 tiles, 67 against 74 us). Results do not depend on the tile.
+static TileKernel w8a16_tile_kernel(int64_t M, int64_t N) {
+  const int64_t cus = compute_units();
+  auto count = [M, N](int64_t bn, int64_t bm) { return ((N + bn - 1) / bn) * ((M + bm - 1) / bm); };
+  if (count(64, 64) <= cus) return {reinterpret_cast<const void*>(&w8a16_ring_kernel<2, 2, 1, 1, 4>), 64, 64, 256, 3};
+  if (count(128, 64) <= cus)
+    return {reinterpret_cast<const void*>(&w8a16_ring_kernel<4, 2, 1, 1, 4>), 128, 64, 512, 2};
+  const int64_t pairs = count(128, 128), rem = pairs % (2 * cus);
+  const double pair = 0.64 * (double)(pairs / (2 * cus)) + (rem == 0 ? 0.0 : rem <= cus ? 0.39 : 0.64);
+  if (pair < (double)((count(256, 256) + cus - 1) / cus))
+    return {reinterpret_cast<const void*>(&w8a16_ring_kernel<4, 2, 1, 2, 3>), 128, 128, 512, 2};
+  return {reinterpret_cast<const void*>(&w8a16_gemm_kernel), 256, 256, kFThreads, 1};
+}
+
 static int w8a16_mm(const uint16_t* x, int64_t M, int64_t K, int64_t xs, const uint8_t* w8, int64_t N,
                     const float* sw, int64_t sw_count, void* y, int64_t ys, hipStream_t s) {
   FLW_REQUIRE(x && w8 && sw && y, FLW_E_INVALID, "null pointer argument");
@@ -1580,12 +1707,13 @@ static int w8a16_mm(const uint16_t* x, int64_t M, int64_t K, int64_t xs, const u
   p.y = static_cast<uint16_t*>(y); p.ys = ys;
   p.M = (int)M; p.N = (int)N; p.K = (int)K;
   p.lds_epi = N % 8 == 0 && ys % 8 == 0 && ((uintptr_t)y & 15) == 0;
-  p.tiles_n = (int)((N + kFBN - 1) / kFBN);
-  p.tiles_m = (int)((M + kFBM - 1) / kFBM);
-  const int64_t tiles = (int64_t)p.tiles_n * p.tiles_m;
-  FLW_REQUIRE(tiles <= 0x7FFFFFFF, FLW_E_UNSUPPORTED, "grid too large");
-  const int64_t grid = tiles < compute_units() ? tiles : compute_units();
-  (void)launch_timed(reinterpret_cast<const void*>(&w8a16_gemm_kernel), dim3((unsigned)grid), dim3(kFThreads), s, p);
+  const TileKernel k = w8a16_tile_kernel(M, N);
+  const int64_t tiles_n = (N + k.bn - 1) / k.bn, tiles_m = (M + k.bm - 1) / k.bm;
+  p.tiles_n = (int)tiles_n;
+  p.tiles_m = (int)tiles_m;
+  const int64_t tiles = tiles_n * tiles_m, slots = (int64_t)compute_units() * k.per_cu;
+  FLW_REQUIRE(tiles <= 0x7FFFFFFF - slots, FLW_E_UNSUPPORTED, "grid too large");
+  (void)launch_timed(k.fn, dim3((unsigned)(tiles < slots ? tiles : slots)), dim3((unsigned)k.threads), s, p);
   return check_launch("flw_fp8_linear (W8A16)");
 }
 

@@ -98,3 +98,26 @@ def test_transform_epilogue_does_not_depend_on_the_tile(D):
         outs[m] = y
     for m, y in outs.items():
         assert torch.equal(y, outs[M][:m]), m
+
+
+@pytest.mark.parametrize("K", [64, 128, 192, 448, 1024])
+@pytest.mark.parametrize("N", [1024, 1004])
+def test_w8a16_rows_do_not_depend_on_the_tile(N, K):
+    """flw_fp8_linear (W8A16): 1020 rows take 64 x 64 tiles, 2000 128 x 64, 4100 128 x 128, all 16380
+    (256 tiles of 256 x 256) the large ones; x with a row stride past K."""
+    from flower_amd import _lib as L
+    lb = L.load()
+    M = 16380
+    _, w8, _, sw = _operands(1, N, K)
+    x = torch.randn(M, K + 8, device="cuda").to(torch.bfloat16)
+    outs = {}
+    for m in (M, 1, 63, 65, 1020, 2000, 4100):
+        y = torch.full((m, N), 7.0, dtype=torch.bfloat16, device="cuda")
+        L.check(lb.flw_fp8_linear(x.data_ptr(), m, K, K + 8, w8.data_ptr(), N, sw.data_ptr(), N, L.GEMM_W8A16,
+                                  y.data_ptr(), N, None, 0, L.stream_of(y)), "w8a16")
+        outs[m] = y
+    for m, y in outs.items():
+        assert torch.equal(y, outs[M][:m]), m
+    ref = x[:64, :K].double() @ (w8.view(torch.float8_e4m3fn).double() * sw[:, None].double()).t().contiguous()
+    d = (outs[M][:64].double() - ref).abs()
+    assert (d <= 2.0 ** -7 * ref.abs() + 1e-3 * ref.pow(2).mean().sqrt()).all()
