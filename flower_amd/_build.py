@@ -2,8 +2,9 @@
 
     python -m flower_amd._build          # compile all HIP sources into flower_amd/libflower_amd.so
 
-The product: one shared object, C ABI only (include/flower_amd.h). Beside it, and never linked
-into it, the diagnostics library flower_amd/libflower_amd_diag.so (csrc/diag/flw_diag.h: device
+The product: one shared object, C ABI only (include/flower_amd.h), and flower_amd/_native.so, the
+Python extension over it that holds the operators' host bodies (csrc/native/flw_host.cpp, host
+compiler, linked against torch and libflower_amd.so). Beside them, and never linked into them, the diagnostics library flower_amd/libflower_amd_diag.so (csrc/diag/flw_diag.h: device
 arithmetic checks and the issue-cost probe that tests and bench.py load). Every HIP source is
 compiled with packed FP32 instructions disabled (``-target-feature -packed-fp32-ops``); sources
 compile in parallel into ``_build/`` and are linked with ``hipcc -shared``.
@@ -25,6 +26,8 @@ DIAG_LIB = os.path.join(HERE, "libflower_amd_diag.so")
 SOURCES = ["flw_error.hip", "flw_quant.hip", "flw_swa.hip", "flw_swa_bf16.hip", "flw_gemm.hip", "flw_heads.hip", "flw_norm_act.hip"]
 # The diagnostics library: its own source plus its own copy of the error / timing state.
 DIAG_SOURCES = ["diag/flw_diag.hip"]
+NATIVE = os.path.join(HERE, "_native.so")
+NATIVE_SOURCE = os.path.join(CSRC, "native", "flw_host.cpp")
 ARCH = os.environ.get("FLW_OFFLOAD_ARCH", "gfx950")
 
 COMMON = [
@@ -68,12 +71,25 @@ def _run_all(cmds, verbose):
         raise RuntimeError("\n".join(errors))
 
 
+def _native_cmd(out: str) -> list:
+    import sysconfig
+
+    import torch
+    from torch.utils import cpp_extension
+    libdir = os.path.join(os.path.dirname(torch.__file__), "lib")
+    inc = [*cpp_extension.include_paths(), sysconfig.get_paths()["include"]]
+    return [shutil.which("g++") or "g++", "-O2", "-std=c++17", "-fPIC", "-shared", "-fvisibility=hidden",
+            f"-D_GLIBCXX_USE_CXX11_ABI={int(torch._C._GLIBCXX_USE_CXX11_ABI)}", *(f"-I{d}" for d in inc), NATIVE_SOURCE,
+            "-o", out, "-L", HERE, "-l:libflower_amd.so", "-L", libdir, "-lc10", "-ltorch_cpu", "-ltorch_python",
+            "-Wl,-rpath,$ORIGIN"]
+
+
 def _obj(source: str) -> str:
     return os.path.join(OBJDIR, os.path.basename(source).replace(".hip", ".o"))
 
 
 def build(verbose: bool = False) -> str:
-    """Compile every source and link both libraries; returns the product library's path."""
+    """Compile every source, link both libraries and the extension; returns the product library's path."""
     os.makedirs(OBJDIR, exist_ok=True)
     cc = hipcc()
     cmds = [[cc, *COMMON, *PER_SOURCE.get(s, []), "-c", os.path.join(CSRC, s), "-o", _obj(s)]
@@ -85,6 +101,8 @@ def build(verbose: bool = False) -> str:
     _run_all(links, verbose)
     for lib in (LIB, DIAG_LIB):
         os.replace(lib + ".tmp", lib)
+    _run_all([_native_cmd(NATIVE + ".tmp")], verbose)
+    os.replace(NATIVE + ".tmp", NATIVE)
     return LIB
 
 

@@ -143,6 +143,7 @@ SIGNATURES = {
 }
 
 # The diagnostics library (flower_amd/csrc/diag/flw_diag.h): instruments for tests and bench.py.
+NATIVE_PATH = os.path.join(os.path.dirname(os.path.abspath(__file__)), "_native.so")
 DIAG_LIB_PATH = os.path.join(_HERE, "libflower_amd_diag.so")
 DIAG_SIGNATURES = {
     "flw_last_error": (c_char_p, []),
@@ -225,7 +226,24 @@ def dtype_code(dt: torch.dtype) -> int:
 
 
 def stream_of(t: torch.Tensor) -> int:
-    return torch.cuda.current_stream(t.device).cuda_stream
+    # torch.cuda.current_stream(t.device).cuda_stream without building a Stream object (2.1 us)
+    return torch._C._cuda_getCurrentRawStream(t.get_device())
+
+
+_native_mod = None
+
+
+def native():
+    """flower_amd._native: the operators' allocate-and-launch bodies in C++ (csrc/native/flw_host.cpp),
+    over the same C ABI; they raise ValueError / FlowerError as ``check`` does."""
+    global _native_mod
+    if _native_mod is None:
+        load()
+        if not os.path.exists(NATIVE_PATH):
+            raise RuntimeError(f"_native.so is not built ({NATIVE_PATH}); run `python -m flower_amd._build`")
+        from . import _native
+        _native_mod = _native
+    return _native_mod
 
 
 def ptr(t: torch.Tensor | None) -> int | None:
@@ -240,5 +258,5 @@ def workspace(nbytes: int, device) -> torch.Tensor:
     return torch.empty(max(int(nbytes), 256), dtype=torch.uint8, device=device)
 
 
-__all__ = ["load", "load_diag", "check", "require_gpu", "dtype_code", "stream_of", "ptr", "i64s", "workspace",
+__all__ = ["load", "load_diag", "native", "check", "require_gpu", "dtype_code", "stream_of", "ptr", "i64s", "workspace",
            "GRANULARITY", "SIGNATURES", "LIB_PATH", "DIAG_SIGNATURES", "DIAG_LIB_PATH"]

@@ -94,18 +94,12 @@ class _QkvHeadsFn(torch.autograd.Function):
 
     @staticmethod
     def forward(ctx, y, num_heads, norm, eps, cos, sin):
-        lib = _lib.load()
         B, T, C = y.shape
-        D = C // (3 * num_heads)
         if y.stride(-1) != 1 or y.stride(0) != T * y.stride(1) or y.stride(1) % 8 or y.data_ptr() % 16:
             y = y.contiguous()
-        q, k, v = (torch.empty((B, num_heads, T, D), dtype=y.dtype, device=y.device) for _ in range(3))
-        rc = lib.flw_qkv_heads_fwd(y.data_ptr(), B, T, num_heads, D, y.stride(1), int(norm), float(eps),
-                                   cos.data_ptr(), sin.data_ptr(), q.data_ptr(), k.data_ptr(), v.data_ptr(),
-                                   _lib.stream_of(y))
-        _lib.check(rc, "qkv_heads")
+        q, k, v = _lib.native().qkv_heads_fwd(y, B, T, num_heads, norm, eps, cos, sin, y.stride(1), _lib.stream_of(y))
         ctx.save_for_backward(y, cos, sin)
-        ctx.meta = (num_heads, norm, eps, D)
+        ctx.meta = (num_heads, norm, eps, C // (3 * num_heads))
         return q, k, v
 
     @staticmethod
@@ -115,12 +109,7 @@ class _QkvHeadsFn(torch.autograd.Function):
         B, T, C = y.shape
         grads = [(g if g is not None else torch.zeros((B, H, T, D), dtype=y.dtype, device=y.device))
                  .to(y.dtype).contiguous() for g in (dq, dk, dv)]
-        dy = torch.empty((B, T, C), dtype=y.dtype, device=y.device)
-        lib = _lib.load()
-        rc = lib.flw_qkv_heads_bwd(y.data_ptr(), B, T, H, D, y.stride(1), int(norm), float(eps), cos.data_ptr(),
-                                   sin.data_ptr(), grads[0].data_ptr(), grads[1].data_ptr(), grads[2].data_ptr(),
-                                   dy.data_ptr(), C, None, None, 0, _lib.stream_of(y))
-        _lib.check(rc, "qkv_heads backward")
+        dy = _lib.native().qkv_heads_bwd(y, B, T, H, norm, eps, cos, sin, y.stride(1), *grads, _lib.stream_of(y))
         return dy, None, None, None, None, None
 
 

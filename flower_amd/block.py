@@ -53,17 +53,9 @@ def _rows(t: torch.Tensor) -> torch.Tensor:
 def _rmsnorm_backward(x2, weight, eps, dh, dres, shape):
     """(dx, dweight) of RMSNorm on the saved rows x2 [rows, cols] for the gradient dh; dres (or None):
     the gradient x2 receives along the residual stream, added in the same pass (flw_rmsnorm_bwd)."""
-    rows, cols = x2.shape
-    lib = _lib.load()
     d2 = _rows(dh.to(x2.dtype))
     r2 = _rows(dres.to(x2.dtype)) if dres is not None else None
-    dx = torch.empty((rows, cols), dtype=x2.dtype, device=x2.device)
-    dw = torch.empty((cols,), dtype=weight.dtype, device=weight.device)
-    ws = _lib.workspace(lib.flw_rmsnorm_bwd_workspace_bytes(rows, cols), x2.device)
-    _lib.check(lib.flw_rmsnorm_bwd(x2.data_ptr(), rows, cols, x2.stride(0), weight.data_ptr(), eps,
-                                   d2.data_ptr(), d2.stride(0), _lib.ptr(r2), r2.stride(0) if r2 is not None else 0,
-                                   dx.data_ptr(), cols, dw.data_ptr(), ws.data_ptr(), ws.numel(),
-                                   _lib.stream_of(x2)), "RMSNorm backward")
+    dx, dw = _lib.native().rmsnorm_bwd(x2, weight, eps, d2, r2, _lib.stream_of(x2))
     return dx.view(shape), dw
 
 
@@ -74,12 +66,8 @@ class _RMSNormFn(torch.autograd.Function):
 
     @staticmethod
     def forward(ctx, x, weight, eps):
-        lib = _lib.load()
         x2 = _rows(x)
-        rows, cols = x2.shape
-        h = torch.empty(x.shape, dtype=x.dtype, device=x.device)
-        _lib.check(lib.flw_rmsnorm_fwd(x2.data_ptr(), rows, cols, x2.stride(0), weight.data_ptr(), float(eps),
-                                       h.data_ptr(), cols, _lib.stream_of(x)), "RMSNorm")
+        h, _ = _lib.native().rmsnorm_fwd(x2, None, weight, float(eps), x.shape, _lib.stream_of(x))
         ctx.save_for_backward(x2, weight)
         ctx.eps, ctx.shape = float(eps), x.shape
         return h
@@ -119,14 +107,7 @@ class _AddRMSNormFn(torch.autograd.Function):
 
     @staticmethod
     def forward(ctx, x, a, weight, eps):
-        lib = _lib.load()
-        x2, a2 = _rows(x), _rows(a)
-        rows, cols = x2.shape
-        s = torch.empty((rows, cols), dtype=x.dtype, device=x.device)
-        h = torch.empty(x.shape, dtype=x.dtype, device=x.device)
-        _lib.check(lib.flw_add_rmsnorm_fwd(x2.data_ptr(), a2.data_ptr(), rows, cols, x2.stride(0), a2.stride(0),
-                                           weight.data_ptr(), float(eps), s.data_ptr(), cols, h.data_ptr(), cols,
-                                           _lib.stream_of(x)), "residual add + RMSNorm")
+        h, s = _lib.native().rmsnorm_fwd(_rows(x), _rows(a), weight, float(eps), x.shape, _lib.stream_of(x))
         ctx.save_for_backward(s, weight)
         ctx.eps, ctx.shape = float(eps), x.shape
         return s.view(x.shape), h
@@ -146,12 +127,8 @@ class _SwiGLUFn(torch.autograd.Function):
 
     @staticmethod
     def forward(ctx, gate, up):
-        lib = _lib.load()
         g2, u2 = _rows(gate), _rows(up)
-        rows, cols = g2.shape
-        h = torch.empty(gate.shape, dtype=gate.dtype, device=gate.device)
-        _lib.check(lib.flw_swiglu_fwd(g2.data_ptr(), u2.data_ptr(), rows, cols, g2.stride(0), u2.stride(0),
-                                      h.data_ptr(), cols, None, None, 0, _lib.stream_of(gate)), "SwiGLU")
+        h, _ = _lib.native().swiglu_fwd(g2, u2, False, gate.shape, _lib.stream_of(gate))
         ctx.save_for_backward(g2, u2)
         ctx.shape = gate.shape
         return h
@@ -159,14 +136,7 @@ class _SwiGLUFn(torch.autograd.Function):
     @staticmethod
     def backward(ctx, dh):
         g2, u2 = ctx.saved_tensors
-        rows, cols = g2.shape
-        lib = _lib.load()
-        d2 = _rows(dh.to(g2.dtype))
-        dg = torch.empty((rows, cols), dtype=g2.dtype, device=g2.device)
-        du = torch.empty((rows, cols), dtype=g2.dtype, device=g2.device)
-        _lib.check(lib.flw_swiglu_bwd(g2.data_ptr(), u2.data_ptr(), rows, cols, g2.stride(0), u2.stride(0),
-                                      d2.data_ptr(), d2.stride(0), dg.data_ptr(), du.data_ptr(), cols, None, None, 0,
-                                      _lib.stream_of(g2)), "SwiGLU backward")
+        dg, du, _ = _lib.native().swiglu_bwd(g2, u2, _rows(dh.to(g2.dtype)), False, _lib.stream_of(g2))
         return dg.view(ctx.shape), du.view(ctx.shape)
 
 
@@ -181,9 +151,8 @@ class _Fp8GatedFn(torch.autograd.Function):
     @staticmethod
     def forward(ctx, x, w_gate, w_up, gate_mod, up_mod):
         from . import precision as P
-        lib = _lib.load()
         x2 = _rows(x)
-        M, K = x2.shape
+        M = x2.shape[0]
         H = gate_mod.out_features
         ld = ((M + 127) // 128) * 128
         x8, x8t, sx = P._quantize_tensorwise_t(x2, ld)
@@ -191,11 +160,7 @@ class _Fp8GatedFn(torch.autograd.Function):
         wu8, swu, wu8t = up_mod.tensorwise_codes()
         g = P.scaled_mm_plain(x8, sx, wg8, swg)
         u = P.scaled_mm_plain(x8, sx, wu8, swu)
-        h = torch.empty((M, H), dtype=x.dtype, device=x.device)
-        amax = torch.empty(1, dtype=torch.int32, device=x.device)
-        ws = _lib.workspace(lib.flw_swiglu_amax_workspace_bytes(M, H), x.device)
-        _lib.check(lib.flw_swiglu_fwd(g.data_ptr(), u.data_ptr(), M, H, H, H, h.data_ptr(), H, amax.data_ptr(),
-                                      ws.data_ptr(), ws.numel(), _lib.stream_of(x)), "SwiGLU")
+        h, amax = _lib.native().swiglu_fwd(g, u, True, g.shape, _lib.stream_of(x))
         ctx.save_for_backward(g, u, x8t, sx, wg8, swg, wu8, swu, wg8t, wu8t)
         ctx.mods, ctx.x_shape, ctx.ld = (gate_mod, up_mod), x.shape, ld
         ctx.mark_non_differentiable(amax)
@@ -211,14 +176,7 @@ class _Fp8GatedFn(torch.autograd.Function):
         gate_mod, up_mod = ctx.mods
         M, H = g.shape
         lib = _lib.load()
-        d2 = _rows(dh.to(g.dtype))
-        dg = torch.empty((M, H), dtype=g.dtype, device=g.device)
-        du = torch.empty((M, H), dtype=g.dtype, device=g.device)
-        amax = torch.empty(2, dtype=torch.int32, device=g.device)
-        ws = _lib.workspace(lib.flw_swiglu_amax_workspace_bytes(M, H), g.device)
-        _lib.check(lib.flw_swiglu_bwd(g.data_ptr(), u.data_ptr(), M, H, H, H, d2.data_ptr(), d2.stride(0),
-                                      dg.data_ptr(), du.data_ptr(), H, amax.data_ptr(), ws.data_ptr(), ws.numel(),
-                                      _lib.stream_of(g)), "SwiGLU backward")
+        dg, du, amax = _lib.native().swiglu_bwd(g, u, _rows(dh.to(g.dtype)), True, _lib.stream_of(g))
         dg8, dg8t, sdg = P._quantize_tensorwise_t(dg, ctx.ld, amax[0:1])
         du8, du8t, sdu = P._quantize_tensorwise_t(du, ctx.ld, amax[1:2])
 
@@ -369,7 +327,7 @@ class Fp8DecoderBlock(nn.Module):
         maxima "amax" of q', k', v, without it the attention operands "q8" / "k8" / "v_tiles" /
         "scales"; the attention output "attn", "x1" and the FF1 output "f". The kernels and the
         result are the same."""
-        lib = _lib.load()
+        native = _lib.native()
         B, T, d = x.shape
         M = B * T
         dev = x.device
@@ -379,41 +337,19 @@ class Fp8DecoderBlock(nn.Module):
             x2 = x2.contiguous()
         qkv_l, out_l, ff1_l, ff2_l = self._linears()
 
-        def codes_of(kind, src, cols, norm=None, h_name=None):
-            c = torch.empty((M, cols), dtype=torch.uint8, device=dev)
-            sc = torch.empty(M, dtype=torch.float32, device=dev)
+        def act_codes(src, h_name, norm=None):
             h = None
-            if trace is not None and h_name is not None:
-                h = trace[h_name] = torch.empty((M, cols), dtype=torch.bfloat16, device=dev)
-            hp = None if h is None else h.data_ptr()
-            if kind == "rmsnorm":
-                rc = lib.flw_rmsnorm_quant_rows_e4m3(src.data_ptr(), M, cols, cols, norm.weight.data_ptr(),
-                                                     float(norm.eps), c.data_ptr(), sc.data_ptr(), hp, stream)
-            elif kind == "gelu":
-                rc = lib.flw_gelu_quant_rows_e4m3(src.data_ptr(), M, cols, cols, c.data_ptr(), sc.data_ptr(),
-                                                  hp, stream)
-            else:
-                rc = lib.flw_quant_rows_e4m3(src.data_ptr(), _lib.BF16, M, cols, cols, c.data_ptr(),
-                                             sc.data_ptr(), stream)
-            _lib.check(rc, kind)
-            return c, sc
+            if trace is not None:
+                h = trace[h_name] = torch.empty(src.shape, dtype=torch.bfloat16, device=dev)
+            return native.act_quant_rows(src, None if norm is None else norm.weight,
+                                         0.0 if norm is None else float(norm.eps), h, stream)
 
         def linear(codes, sc, lin, residual=None):
             w8, ws = lin.weight_codes()
-            N, K = w8.shape
-            y = torch.empty((M, N), dtype=torch.bfloat16, device=dev)
-            if residual is None:
-                rc = lib.flw_fp8_scaled_mm(codes.data_ptr(), M, K, w8.data_ptr(), N, sc.data_ptr(), M,
-                                           ws.data_ptr(), ws.numel(), y.data_ptr(), N, stream)
-            else:
-                rc = lib.flw_fp8_scaled_mm_residual(codes.data_ptr(), M, K, w8.data_ptr(), N, sc.data_ptr(), M,
-                                                    ws.data_ptr(), ws.numel(), y.data_ptr(), N,
-                                                    residual.data_ptr(), residual.stride(0), stream)
-            _lib.check(rc, "fp8 linear")
-            return y
+            return native.scaled_mm(codes, sc, w8, ws, residual, False, stream)
 
         att = self.attn
-        c1, s1 = codes_of("rmsnorm", x2, d, self.ln1, "h1")
+        c1, s1 = act_codes(x2, "h1", self.ln1)
         cos, sin = att.rope.tables(T, torch.bfloat16, dev)
         qk_norm = att.qk_norm is not None
         eps = att.qk_norm.eps if qk_norm else 0.0
@@ -429,13 +365,7 @@ class Fp8DecoderBlock(nn.Module):
             # (K % 128 == 0, operands < 2^32 bytes) carries this epilogue; other shapes take the
             # quantiser pair below.
             w8, ws = qkv_l.weight_codes()
-            N, K = w8.shape
-            qkv = torch.empty((M, N), dtype=torch.bfloat16, device=dev)
-            amax = torch.empty(N // att.head_dim, dtype=torch.int32, device=dev)
-            _lib.check(lib.flw_fp8_scaled_mm_qk_norm_rope_amax(
-                c1.data_ptr(), M, K, w8.data_ptr(), N, s1.data_ptr(), M, ws.data_ptr(), ws.numel(), qkv.data_ptr(),
-                N, att.head_dim, 2 * d, int(qk_norm), float(eps), cos.data_ptr(), sin.data_ptr(), T, amax.data_ptr(),
-                stream), "qkv + qk-norm + rope + amax")
+            qkv, amax = native.qkv_norm_rope_amax(c1, s1, w8, ws, att.head_dim, qk_norm, float(eps), cos, sin, T, stream)
             qkv = qkv.view(B, T, 3 * d)
             q, k, v = (att._split(t) for t in qkv.chunk(3, dim=-1))
             fp8_swa_attention_forward(q, k, v, window, granularity="head", out=a_heads, amax=amax)
@@ -451,11 +381,11 @@ class Fp8DecoderBlock(nn.Module):
             fp8_swa_attention_from_codes(*res[:4], window, granularity=att.granularity, out=a_heads)
             if trace is not None:
                 trace.update(q=res[4], k=res[5], q8=res[0], k8=res[1], v_tiles=res[2], scales=res[3])
-        ca, sa = codes_of("plain", a.view(M, d), d)
+        ca, sa = native.quant_rows(a.view(M, d), "plain", stream)
         x1 = linear(ca, sa, out_l, residual=x2)
-        c2, s2 = codes_of("rmsnorm", x1, d, self.ln2, "h2")
+        c2, s2 = act_codes(x1, "h2", self.ln2)
         f = linear(c2, s2, ff1_l)
-        cg, sg = codes_of("gelu", f, f.shape[1], h_name="hg")
+        cg, sg = act_codes(f, "hg")
         if trace is not None:
             trace.update(c1=c1, s1=s1, qkv=qkv, attn=a, ca=ca, sa=sa, x1=x1, c2=c2, s2=s2, f=f, cg=cg, sg=sg)
         return linear(cg, sg, ff2_l, residual=x1).view(B, T, d)

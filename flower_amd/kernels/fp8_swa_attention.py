@@ -161,7 +161,7 @@ def fp8_swa_attention_forward(
     """
     del block_m, block_n, num_warps, num_stages
     try:
-        lib = _lib.load()
+        _lib.load()
     except RuntimeError as e:
         raise RuntimeError(f"fp8_swa_attention_forward requires the HIP library: {e}") from e
     if q.requires_grad or k.requires_grad or v.requires_grad:
@@ -182,24 +182,11 @@ def fp8_swa_attention_forward(
     _lib.require_gpu(q, k, v)
     if q.numel() == 0:
         return torch.empty_like(q)
-    dt = _lib.dtype_code(q.dtype)
-    q, sq = _prepare(q)
-    k, sk = _prepare(k)
-    v, sv = _prepare(v)
-    if out is None:
-        out = torch.empty((B, H, T, D), device=q.device, dtype=q.dtype)
-    elif (out.shape != (B, H, T, D) or out.dtype != q.dtype or out.device != q.device
-          or out.stride(-1) != 1):
+    _lib.dtype_code(q.dtype)
+    if out is not None and (out.shape != (B, H, T, D) or out.dtype != q.dtype or out.device != q.device
+                            or out.stride(-1) != 1):
         raise ValueError("out must be a (B, H, T, D) tensor of q's dtype and device with D contiguous")
-    so = out.stride()[:3]
-    ws = _lib.workspace(lib.flw_fp8_swa_workspace_bytes(B, H, T, D), q.device)
-    strides = _lib.i64s(*sq, *sk, *sv, *so)
-    if amax is None:
-        rc = lib.flw_fp8_swa_attention_forward(
-            q.data_ptr(), k.data_ptr(), v.data_ptr(), dt, strides, B, H, T, D, int(window),
-            _lib.GRANULARITY[granularity], out.data_ptr(), None, ws.data_ptr(), ws.numel(),
-            _lib.stream_of(q))
-    else:
+    if amax is not None:
         groups = {"tensor": 1, "head": H, "bh": B * H}[granularity]
         if amax.dtype == torch.float32:
             amax = amax.view(torch.int32)
@@ -207,12 +194,8 @@ def fp8_swa_attention_forward(
                 or not amax.is_contiguous()):
             raise ValueError(f"amax must be a contiguous float32 tensor (or its int32 bit patterns) of "
                              f"{3 * groups} elements on q's device")
-        rc = lib.flw_fp8_swa_attention_forward_amax(
-            q.data_ptr(), k.data_ptr(), v.data_ptr(), dt, strides, B, H, T, D, int(window),
-            _lib.GRANULARITY[granularity], amax.data_ptr(), out.data_ptr(), None, ws.data_ptr(), ws.numel(),
-            _lib.stream_of(q))
-    _lib.check(rc, "fp8_swa_attention_forward")
-    return out
+    return _lib.native().fp8_swa_forward(q, k, v, int(window), _lib.GRANULARITY[granularity], out, amax,
+                                         _lib.stream_of(q))
 
 
 def reference_swa_attention(
@@ -411,56 +394,18 @@ class _Fp8SwaAttention(torch.autograd.Function):
 
     @staticmethod
     def forward(ctx, q, k, v, window, granularity):
-        lib = _lib.load()
-        B, H, T, D = q.shape
-        dt = _lib.dtype_code(q.dtype)
-        q, sq = _prepare(q.detach())
-        k, sk = _prepare(k.detach())
-        v, sv = _prepare(v.detach())
-        G = _group_count(granularity, B, H)
-        dev = q.device
-        q8 = torch.empty((B, H, T, D), dtype=torch.uint8, device=dev)
-        k8 = torch.empty_like(q8)
-        vt = torch.empty(lib.flw_vtile_bytes(B, H, T, D), dtype=torch.uint8, device=dev)
-        scales = torch.empty(3 * G, dtype=torch.float32, device=dev)
-        ws = _lib.workspace(3 * lib.flw_quant_workspace_bytes(B, H, T, D), dev)
-        stream = _lib.stream_of(q)
-        _lib.check(lib.flw_quant_qkv_e4m3(q.data_ptr(), k.data_ptr(), v.data_ptr(), dt, B, H, T, D,
-                                          _lib.i64s(*sq, *sk, *sv), _lib.GRANULARITY[granularity], q8.data_ptr(),
-                                          k8.data_ptr(), vt.data_ptr(), scales.data_ptr(), ws.data_ptr(),
-                                          ws.numel(), stream), "fp8_swa_attention (quantise)")
-        out = torch.empty((B, H, T, D), dtype=q.dtype, device=dev)
-        s8 = _lib.i64s(H * T * D, T * D, D)
-        base = scales.data_ptr()
-        rc = lib.flw_fp8_swa_fwd(q8.data_ptr(), s8, k8.data_ptr(), s8, vt.data_ptr(), base, base + 4 * G,
-                                 base + 8 * G, _lib.GRANULARITY[granularity], out.data_ptr(), dt,
-                                 _lib.i64s(*out.stride()[:3]), B, H, T, D, int(window), stream)
-        _lib.check(rc, "fp8_swa_attention (forward)")
+        out, q8, k8, vt, scales = _lib.native().fp8_swa_train_fwd(q, k, v, int(window), _lib.GRANULARITY[granularity],
+                                                                  _lib.stream_of(q))
         ctx.save_for_backward(q8, k8, vt, scales)
-        ctx.window, ctx.granularity, ctx.G, ctx.dtype = int(window), granularity, G, q.dtype
+        ctx.window, ctx.granularity, ctx.dtype = int(window), granularity, q.dtype
         return out
 
     @staticmethod
     def backward(ctx, dout):
-        lib = _lib.load()
         q8, k8, vt, scales = ctx.saved_tensors
-        B, H, T, D = q8.shape
-        G, gran = ctx.G, ctx.granularity
-        qd = dequantize_e4m3(q8, scales[:G], (B, H, T, D), gran)
-        kd = dequantize_e4m3(k8, scales[G:2 * G], (B, H, T, D), gran)
-        vd = dequantize_e4m3(vt, scales[2 * G:], (B, H, T, D), gran, layout="vtile")
-        stream = _lib.stream_of(qd)
-        ob = torch.empty_like(qd)
-        lse = torch.empty((B, H, T), dtype=torch.float32, device=qd.device)
-        _lib.check(lib.flw_swa_bf16_fwd(qd.data_ptr(), kd.data_ptr(), vd.data_ptr(), B, H, T, D, ctx.window,
-                                        ob.data_ptr(), lse.data_ptr(), stream), "fp8_swa_attention (recompute)")
-        do = dout.to(torch.bfloat16).contiguous()
-        dq, dk, dv = torch.empty_like(qd), torch.empty_like(kd), torch.empty_like(vd)
-        ws = _lib.workspace(lib.flw_swa_bf16_bwd_workspace_bytes(B, H, T, D), q8.device)
-        _lib.check(lib.flw_swa_bf16_bwd(qd.data_ptr(), kd.data_ptr(), vd.data_ptr(), ob.data_ptr(), do.data_ptr(),
-                                        lse.data_ptr(), B, H, T, D, ctx.window, dq.data_ptr(), dk.data_ptr(),
-                                        dv.data_ptr(), ws.data_ptr(), ws.numel(), stream),
-                   "fp8_swa_attention (backward)")
+        dq, dk, dv = _lib.native().fp8_swa_train_bwd(q8, k8, vt, scales, dout.to(torch.bfloat16).contiguous(),
+                                                     ctx.window, _lib.GRANULARITY[ctx.granularity],
+                                                     _lib.stream_of(q8))
         dt = ctx.dtype
         return dq.to(dt), dk.to(dt), dv.to(dt), None, None
 

@@ -29,40 +29,26 @@ _DQ_CFG = (128, 64, 4, 2)
 class _SlidingWindowAttention(torch.autograd.Function):
     @staticmethod
     def forward(ctx, q, k, v, window, token_major=False):
-        lib = _lib.load()
-        B, H, T, D = q.shape
         q, k, v = q.contiguous(), k.contiguous(), v.contiguous()
         # token_major: O stored (B, T, H, D) and returned as its (B, H, T, D) view, so that the
         # caller's transpose(1, 2).reshape(B, T, H D) is a view (no copy); the backward then takes
         # dO as that layout's view too.
-        out = torch.empty((B, T, H, D) if token_major else (B, H, T, D), dtype=q.dtype, device=q.device)
-        lse = torch.empty((B, H, T), device=q.device, dtype=torch.float32)
-        layout = _lib.LAYOUT_BTHD if token_major else _lib.LAYOUT_BHTD
-        rc = lib.flw_swa_bf16_fwd_layout(q.data_ptr(), k.data_ptr(), v.data_ptr(), B, H, T, D, int(window),
-                                         out.data_ptr(), layout, lse.data_ptr(), _lib.stream_of(q))
-        _lib.check(rc, "swa_attention forward")
+        out, lse = _lib.native().swa_bf16_fwd(q, k, v, int(window), token_major, "swa_attention forward",
+                                              _lib.stream_of(q))
         ctx.save_for_backward(q, k, v, out, lse)
-        ctx.window, ctx.layout = int(window), layout
+        ctx.window, ctx.token_major = int(window), token_major
         return out.transpose(1, 2) if token_major else out
 
     @staticmethod
     def backward(ctx, do):
-        lib = _lib.load()
         q, k, v, out, lse = ctx.saved_tensors
-        B, H, T, D = q.shape
         if do.dtype != q.dtype:
             do = do.to(q.dtype)
         # dO in the forward's O layout: a view of it when the gradient comes that way (the output
         # projection's gradient, token-major), a copy otherwise
-        do = do.transpose(1, 2).contiguous() if ctx.layout == _lib.LAYOUT_BTHD else do.contiguous()
-        dptr = do.data_ptr()
-        dq, dk, dv = torch.empty_like(q), torch.empty_like(k), torch.empty_like(v)
-        ws = _lib.workspace(lib.flw_swa_bf16_bwd_workspace_bytes(B, H, T, D), q.device)
-        rc = lib.flw_swa_bf16_bwd_layout(q.data_ptr(), k.data_ptr(), v.data_ptr(), out.data_ptr(), dptr,
-                                         ctx.layout, lse.data_ptr(), B, H, T, D, ctx.window, dq.data_ptr(),
-                                         dk.data_ptr(), dv.data_ptr(), ws.data_ptr(), ws.numel(),
-                                         _lib.stream_of(q))
-        _lib.check(rc, "swa_attention backward")
+        do = do.transpose(1, 2).contiguous() if ctx.token_major else do.contiguous()
+        dq, dk, dv = _lib.native().swa_bf16_bwd(q, k, v, out, do, ctx.token_major, lse, ctx.window,
+                                                "swa_attention backward", _lib.stream_of(q))
         return dq, dk, dv, None, None
 
 

@@ -79,73 +79,39 @@ def _compute_units(device) -> int:
     return _CUS[idx]
 
 
-def _quantize_tensorwise(x2: torch.Tensor, out8: torch.Tensor, scale: torch.Tensor) -> None:
-    """One e4m3 scale for the whole matrix x2 [R, C] (bf16 / fp32, rows of stride C' >= C): codes to
-    out8 [R, C]. A contiguous matrix goes to the quantiser as a flat grid of rows of 64 to 1024
-    values (one chunk of 128 such rows per workgroup): the widest rows that still leave two chunks
-    per compute unit, so the passes spread over the GPU whatever the matrix's shape while every
-    quantising workgroup folds as few amax partials as possible (each one reads all of them). The
-    amax, the scale and every code are those of the matrix itself."""
-    lib = _lib.load()
-    R, C = x2.shape
-    n = R * C
-    if x2.is_contiguous() and n % 64 == 0:
-        cols, floor = 64, 2 * _compute_units(x2.device)
-        while cols < 1024 and n % (2 * cols) == 0 and (n // (2 * cols) + 127) // 128 >= floor:
-            cols *= 2
-        rows, ld = n // cols, cols
-    else:
-        rows, cols, ld = R, C, x2.stride(0)
-    ws = _lib.workspace(lib.flw_quant_workspace_bytes(1, 1, rows, cols), x2.device)
-    rc = lib.flw_quant_e4m3(x2.data_ptr(), _lib.dtype_code(x2.dtype), 1, 1, rows, cols, rows * ld, rows * ld,
-                            ld, _lib.SCALE_TENSOR, _lib.LAYOUT_BHTD, out8.data_ptr(), scale.data_ptr(),
-                            ws.data_ptr(), ws.numel(), _lib.stream_of(x2))
-    _lib.check(rc, "tensorwise e4m3")
+def _quantize_tensorwise(x2: torch.Tensor):
+    """(x8 [R, C], scale [1]): one e4m3 scale for the whole matrix x2 [R, C] (bf16 / fp32, rows of
+    stride C' >= C). The amax, the scale and every code are those of the matrix itself whatever grid
+    the native body lays over it."""
+    return _lib.native().quant_tensorwise(x2, _compute_units(x2.device), _lib.stream_of(x2))
 
 
 def quantize_weight(weight: torch.Tensor, recipe: str = "rowwise"):
     """(w8 [N, K] uint8 e4m3 codes, w_scale float32 [N] or [1]) on the weight's device."""
-    lib = _lib.load()
+    _lib.load()
     _lib.require_gpu(weight)
     w = weight.detach()
     if w.dtype not in (torch.float32, torch.bfloat16):
         w = w.to(torch.bfloat16)
     w = w.contiguous()
-    N, K = w.shape
-    w8 = torch.empty((N, K), dtype=torch.uint8, device=w.device)
     if recipe in ("rowwise", "weight_only"):
-        scale = torch.empty(N, dtype=torch.float32, device=w.device)
-        rc = lib.flw_quant_rows_e4m3(w.data_ptr(), _lib.dtype_code(w.dtype), N, K, K, w8.data_ptr(),
-                                     scale.data_ptr(), _lib.stream_of(w))
-        _lib.check(rc, "quantize_weight")
-    elif recipe == "tensorwise":
-        scale = torch.empty(1, dtype=torch.float32, device=w.device)
-        _quantize_tensorwise(w, w8, scale)
-    else:
-        raise RuntimeError(f"training.fp8_recipe must be one of {sorted(RECIPES)}, got {recipe!r}")
-    return w8, scale
+        return _lib.native().quant_rows(w, "quantize_weight", _lib.stream_of(w))
+    if recipe == "tensorwise":
+        return _quantize_tensorwise(w)
+    raise RuntimeError(f"training.fp8_recipe must be one of {sorted(RECIPES)}, got {recipe!r}")
 
 
 def quantize_cols(x2: torch.Tensor, granularity: str, ld: int | None = None):
     """(codes_t [C, ld] uint8, scale float32 [C] or [1]): e4m3 of each column of x2 [R, C] (bf16 or
     fp32, rows contiguous), transposed; rows past R up to ld (a multiple of 16) are coded 0."""
-    lib = _lib.load()
+    _lib.load()
     _lib.require_gpu(x2)
     if x2.dtype not in (torch.float32, torch.bfloat16):
         x2 = x2.to(torch.bfloat16)
-    if x2.stride(-1) != 1 or x2.stride(0) % 8 or x2.data_ptr() % 16:
-        x2 = x2.contiguous()
-    R, C = x2.shape
+    x2 = _lib.native().rows16(x2)
+    R = x2.shape[0]
     ld = ((R + 15) // 16) * 16 if ld is None else ld
-    gran = _lib.SCALE_COLUMN if granularity == "column" else _lib.SCALE_TENSOR
-    out = torch.empty((C, ld), dtype=torch.uint8, device=x2.device)
-    scale = torch.empty(C if gran == _lib.SCALE_COLUMN else 1, dtype=torch.float32, device=x2.device)
-    ws = _lib.workspace(lib.flw_quant_cols_workspace_bytes(R, C), x2.device)
-    rc = lib.flw_quant_cols_e4m3(x2.data_ptr(), _lib.dtype_code(x2.dtype), R, C, x2.stride(0), gran,
-                                 out.data_ptr(), ld, scale.data_ptr(), ws.data_ptr(), ws.numel(),
-                                 _lib.stream_of(x2))
-    _lib.check(rc, "quantize_cols")
-    return out, scale
+    return _lib.native().quant_cols(x2, granularity == "column", ld, _lib.stream_of(x2))
 
 
 def quantize_weight_cols(weight: torch.Tensor, recipe: str = "rowwise"):
@@ -158,34 +124,15 @@ def quantize_weight_cols(weight: torch.Tensor, recipe: str = "rowwise"):
 def _quantize_rows(x2: torch.Tensor, recipe: str):
     """(x8 [M, K], scale [M] or [1]) of a contiguous bf16 / fp32 matrix, per row ("rowwise") or
     per tensor ("tensorwise")."""
-    lib = _lib.load()
-    M, K = x2.shape
-    x8 = torch.empty((M, K), dtype=torch.uint8, device=x2.device)
-    stream = _lib.stream_of(x2)
     if recipe == "rowwise":
-        sx = torch.empty(M, dtype=torch.float32, device=x2.device)
-        rc = lib.flw_quant_rows_e4m3(x2.data_ptr(), _lib.dtype_code(x2.dtype), M, K, x2.stride(0),
-                                     x8.data_ptr(), sx.data_ptr(), stream)
-        _lib.check(rc, "quantize rows")
-    else:
-        sx = torch.empty(1, dtype=torch.float32, device=x2.device)
-        _quantize_tensorwise(x2, x8, sx)
-    return x8, sx
+        return _lib.native().quant_rows(x2, "quantize rows", _lib.stream_of(x2))
+    return _quantize_tensorwise(x2)
 
 
 def scaled_mm(a8: torch.Tensor, sa: torch.Tensor, b8: torch.Tensor, sb: torch.Tensor) -> torch.Tensor:
     """bf16 [M, N] = (a8 [M, K] . b8 [N, K]^T) * sa[m] * sb[n] through flw_fp8_scaled_mm_ws (split
     over K into a workspace when [M, N] has too few output tiles to fill the GPU)."""
-    lib = _lib.load()
-    M, K = a8.shape
-    N = b8.shape[0]
-    y = torch.empty((M, N), dtype=torch.bfloat16, device=a8.device)
-    ws = _lib.workspace(lib.flw_fp8_scaled_mm_workspace_bytes(M, N, K), a8.device)
-    rc = lib.flw_fp8_scaled_mm_ws(a8.data_ptr(), M, K, b8.data_ptr(), N, sa.data_ptr(), sa.numel(),
-                                  sb.data_ptr(), sb.numel(), y.data_ptr(), N, ws.data_ptr(), ws.numel(),
-                                  _lib.stream_of(a8))
-    _lib.check(rc, "fp8_scaled_mm")
-    return y
+    return _lib.native().scaled_mm(a8, sa, b8, sb, None, True, _lib.stream_of(a8))
 
 
 def _quantize_tensorwise_t(x2: torch.Tensor, ld: int, amax: torch.Tensor | None = None):
@@ -194,33 +141,13 @@ def _quantize_tensorwise_t(x2: torch.Tensor, ld: int, amax: torch.Tensor | None 
     (flw_quant_tensor_t_e4m3): the codes of _quantize_tensorwise, and transpose_codes of them.
     amax: x2's |x| maximum as a device fp32 bit pattern from its producer (int32 [1]): then the
     quantise pass alone (flw_quant_tensor_t_e4m3_amax)."""
-    lib = _lib.load()
-    R, C = x2.shape
-    x8 = torch.empty((R, C), dtype=torch.uint8, device=x2.device)
-    x8t = torch.empty((C, ld), dtype=torch.uint8, device=x2.device)
-    sx = torch.empty(1, dtype=torch.float32, device=x2.device)
-    if amax is not None:
-        rc = lib.flw_quant_tensor_t_e4m3_amax(x2.data_ptr(), R, C, x2.stride(0), amax.data_ptr(), x8.data_ptr(), C,
-                                              x8t.data_ptr(), ld, sx.data_ptr(), _lib.stream_of(x2))
-    else:
-        ws = _lib.workspace(lib.flw_quant_tensor_t_workspace_bytes(R, C), x2.device)
-        rc = lib.flw_quant_tensor_t_e4m3(x2.data_ptr(), R, C, x2.stride(0), x8.data_ptr(), C, x8t.data_ptr(), ld,
-                                         sx.data_ptr(), ws.data_ptr(), ws.numel(), _lib.stream_of(x2))
-    _lib.check(rc, "tensorwise e4m3 (rows and columns)")
-    return x8, x8t, sx
+    return _lib.native().quant_tensor_t(x2, ld, amax, _lib.stream_of(x2))
 
 
 def scaled_mm_plain(a8: torch.Tensor, sa: torch.Tensor, b8: torch.Tensor, sb: torch.Tensor) -> torch.Tensor:
     """bf16 [M, N] = (a8 [M, K] . b8 [N, K]^T) * sa * sb through flw_fp8_scaled_mm (never split over
     K): the forward GEMM of fp8_linear_forward's tensorwise route."""
-    lib = _lib.load()
-    M, K = a8.shape
-    N = b8.shape[0]
-    y = torch.empty((M, N), dtype=torch.bfloat16, device=a8.device)
-    rc = lib.flw_fp8_scaled_mm(a8.data_ptr(), M, K, b8.data_ptr(), N, sa.data_ptr(), sa.numel(), sb.data_ptr(),
-                               sb.numel(), y.data_ptr(), N, _lib.stream_of(a8))
-    _lib.check(rc, "fp8_scaled_mm")
-    return y
+    return _lib.native().scaled_mm(a8, sa, b8, sb, None, False, _lib.stream_of(a8))
 
 
 def scaled_mm_residual(a8: torch.Tensor, sa: torch.Tensor, b8: torch.Tensor, sb: torch.Tensor,
@@ -228,28 +155,15 @@ def scaled_mm_residual(a8: torch.Tensor, sa: torch.Tensor, b8: torch.Tensor, sb:
     """bf16 [M, N] = res + bf16((a8 . b8^T) * sa * sb), both terms rounded to bf16 as torch adds a
     Linear's output to a tensor (flw_fp8_scaled_mm_residual; never split over K). res: [M, N] bf16
     rows with a unit column stride."""
-    lib = _lib.load()
-    M, K = a8.shape
-    N = b8.shape[0]
-    y = torch.empty((M, N), dtype=torch.bfloat16, device=a8.device)
-    rc = lib.flw_fp8_scaled_mm_residual(a8.data_ptr(), M, K, b8.data_ptr(), N, sa.data_ptr(), sa.numel(),
-                                        sb.data_ptr(), sb.numel(), y.data_ptr(), N, res.data_ptr(), res.stride(0),
-                                        _lib.stream_of(a8))
-    _lib.check(rc, "fp8_scaled_mm_residual")
-    return y
+    return _lib.native().scaled_mm(a8, sa, b8, sb, res, False, _lib.stream_of(a8))
 
 
 def transpose_codes(c8: torch.Tensor, ld: int | None = None) -> torch.Tensor:
     """[C, ld] uint8: the e4m3 codes c8 [R, C] transposed (ld >= R, a multiple of 16; columns past R
     zero). Under one scale per tensor a matrix's column codes are its row codes, so this gives
     quantize_cols(x, "tensor")'s codes from the row codes without reading x again."""
-    lib = _lib.load()
-    R, C = c8.shape
-    ld = ((R + 15) // 16) * 16 if ld is None else ld
-    out = torch.empty((C, ld), dtype=torch.uint8, device=c8.device)
-    rc = lib.flw_transpose_e4m3(c8.data_ptr(), R, C, c8.stride(0), out.data_ptr(), ld, _lib.stream_of(c8))
-    _lib.check(rc, "transpose codes")
-    return out
+    ld = ((c8.shape[0] + 15) // 16) * 16 if ld is None else ld
+    return _lib.native().transpose_codes(c8, ld, _lib.stream_of(c8))
 
 
 def fp8_linear_backward(g2: torch.Tensor, x2: torch.Tensor, w_cols, recipe: str,
@@ -305,58 +219,33 @@ def fp8_linear_forward(x: torch.Tensor, w8: torch.Tensor, w_scale: torch.Tensor,
     (with return_codes): x's |x| maximum from its producer, which spares that pass its amax pass.
     residual (bf16, x's leading shape by N): returns residual + y as torch's add of the two bf16
     tensors gives it, in the tensorwise GEMM's epilogue (after the GEMM otherwise)."""
-    lib = _lib.load()
+    native = _lib.native()
     _lib.require_gpu(x, w8)
     N, K = w8.shape
     lead = x.shape[:-1]
     x2 = x.reshape(-1, K)
     if x2.dtype != torch.bfloat16:
         x2 = x2.to(torch.bfloat16)
-    if x2.stride(-1) != 1 or x2.stride(0) % 8 or x2.data_ptr() % 16:
-        x2 = x2.contiguous()
+    x2 = native.rows16(x2)
     M = x2.shape[0]
-    y = torch.empty((M, N), dtype=torch.bfloat16, device=x.device)
     if M == 0:
-        return (y.reshape(*lead, N), None, None) if return_codes else y.reshape(*lead, N)
+        y = torch.empty((*lead, N), dtype=torch.bfloat16, device=x.device)
+        return (y, None, None) if return_codes else y
     stream = _lib.stream_of(x2)
-    if recipe == "weight_only":
-        rc = lib.flw_fp8_linear(x2.data_ptr(), M, K, x2.stride(0), w8.data_ptr(), N, w_scale.data_ptr(),
-                                w_scale.numel(), _lib.GEMM_W8A16, y.data_ptr(), N, None, 0, stream)
-        _lib.check(rc, "fp8_linear(weight_only)")
-    elif recipe == "rowwise":
-        ws = _lib.workspace(lib.flw_fp8_linear_workspace_bytes(M, K, _lib.GEMM_A8W8), x.device)
-        rc = lib.flw_fp8_linear(x2.data_ptr(), M, K, x2.stride(0), w8.data_ptr(), N, w_scale.data_ptr(),
-                                w_scale.numel(), _lib.GEMM_A8W8, y.data_ptr(), N, ws.data_ptr(),
-                                ws.numel(), stream)
-        _lib.check(rc, "fp8_linear")
+    if recipe != "tensorwise":
+        y = native.linear(x2, w8, w_scale, recipe == "weight_only", stream).view(*lead, N)
+        return y if residual is None else residual + y
+    ld = ((M + 127) // 128) * 128
+    x8t = None
+    if return_codes and K % 16 == 0:
+        x8, x8t, sx = _quantize_tensorwise_t(x2, ld, x_amax)
     else:
-        x8t = None
-        if return_codes and K % 16 == 0:
-            x8, x8t, sx = _quantize_tensorwise_t(x2, ((M + 127) // 128) * 128, x_amax)
-        else:
-            x8 = torch.empty((M, K), dtype=torch.uint8, device=x.device)
-            sx = torch.empty(1, dtype=torch.float32, device=x.device)
-            _quantize_tensorwise(x2, x8, sx)
-        r2 = None
-        if residual is not None:
-            r2 = residual.reshape(M, N).to(torch.bfloat16)
-            if r2.stride(-1) != 1 or r2.stride(0) % 8 or r2.data_ptr() % 16:
-                r2 = r2.contiguous()
-            rc = lib.flw_fp8_scaled_mm_residual(x8.data_ptr(), M, K, w8.data_ptr(), N, sx.data_ptr(), 1,
-                                                w_scale.data_ptr(), w_scale.numel(), y.data_ptr(), N,
-                                                r2.data_ptr(), r2.stride(0), stream)
-            residual = None
-        else:
-            rc = lib.flw_fp8_scaled_mm(x8.data_ptr(), M, K, w8.data_ptr(), N, sx.data_ptr(), 1,
-                                       w_scale.data_ptr(), w_scale.numel(), y.data_ptr(), N, stream)
-        _lib.check(rc, "fp8_scaled_mm")
-        if return_codes:
-            if x8t is None:
-                x8t = transpose_codes(x8, ((M + 127) // 128) * 128)
-            return y.reshape(*lead, N), x8t, sx
-    if residual is not None:
-        return residual + y.reshape(*lead, N)
-    return y.reshape(*lead, N)
+        x8, sx = _quantize_tensorwise(x2)
+    r2 = native.rows16(residual.reshape(M, N).to(torch.bfloat16)) if residual is not None else None
+    y = native.scaled_mm(x8, sx, w8, w_scale, r2, False, stream).view(*lead, N)
+    if return_codes:
+        return y, (transpose_codes(x8, ld) if x8t is None else x8t), sx
+    return y
 
 
 class _Fp8LinearFn(torch.autograd.Function):
