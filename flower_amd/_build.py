@@ -39,10 +39,12 @@ COMMON = [
 # place instead of copying through AGPRs), and no IEEE mode, since in IEEE mode every fmax operand
 # of the row max is first re-quietened (one extra VALU op per score); NaN inputs still give NaN
 # rows without it. GEMM: accumulators in VGPRs too; in AGPRs every branch of a short K loop moved
-# them to VGPRs and back (64 x 64 tiles at K = 4096: 11.5 against 8.9 us). The other sources keep the
-# compiler's default forms.
+# them to VGPRs and back (64 x 64 tiles at K = 4096: 11.5 against 8.9 us). bf16 attention: the same at
+# head dim 128 (backward 409 -> 342 us at B2 H16 T4096 W1024; the other head dims compile alike). The
+# other sources keep the compiler's default forms.
 VGPR_FORM = ["-mllvm", "-amdgpu-mfma-vgpr-form=1"]
-PER_SOURCE = {"flw_swa.hip": [*VGPR_FORM, "-fno-honor-nans", "-mno-amdgpu-ieee"], "flw_gemm.hip": VGPR_FORM}
+PER_SOURCE = {"flw_swa.hip": [*VGPR_FORM, "-fno-honor-nans", "-mno-amdgpu-ieee"], "flw_gemm.hip": VGPR_FORM,
+              "flw_swa_bf16.hip": VGPR_FORM}
 NOISE = "'-packed-fp32-ops' is not a recognized feature"
 
 

@@ -392,7 +392,7 @@ __global__ __launch_bounds__(256, D == 128 ? 1 : 2) void swa_bf16_dkdv_kernel(Sw
   constexpr int KS = D / 16, NDB = D / 32, NAT = 64 * D * 2;
   __shared__ __align__(16) uint8_t lq[2][NAT];     // Q tile: A operand of S, read transposed for dK
   __shared__ __align__(16) uint8_t ldo[2][NAT];    // dO tile: A operand of dP, read transposed for dV
-  __shared__ __align__(16) float lstat[2][2][64];  // -L log2(e) and Delta of the tile's queries
+  __shared__ __align__(16) float lstat[2][2][64];  // -L log2(e) and -Delta of the tile's queries
   const int tid = threadIdx.x, lane = tid & 63, wave = __builtin_amdgcn_readfirstlane(tid >> 6), h = lane >> 5, kc = lane & 31;
   int bh, nt0;
   band_order(p, true, bh, nt0);
@@ -430,7 +430,7 @@ __global__ __launch_bounds__(256, D == 128 ? 1 : 2) void swa_bf16_dkdv_kernel(Sw
   TileLoadLds<D> tq, tdo;
   tq.init(p.q + slice, T, wave, lane);
   tdo.init(p.dout + o_base(p, bh, D), T, wave, lane, o_ld(p, D));
-  // Wave 0 carries L of the tile's 64 queries (stored as -L log2(e)), wave 1 their Delta; both
+  // Wave 0 carries L of the tile's 64 queries (stored as -L log2(e)), wave 1 their -Delta; both
   // through buffer descriptors over the slice's T values, so queries past T read as 0.
   const __amdgpu_buffer_rsrc_t lrs = __builtin_amdgcn_make_buffer_rsrc(const_cast<float*>(LSE), 0, T * 4, kBufferFlags);
   const __amdgpu_buffer_rsrc_t drs = __builtin_amdgcn_make_buffer_rsrc(const_cast<float*>(DLT), 0, T * 4, kBufferFlags);
@@ -442,7 +442,7 @@ __global__ __launch_bounds__(256, D == 128 ? 1 : 2) void swa_bf16_dkdv_kernel(Sw
   };
   auto store_stat = [&](int buf, float x) __attribute__((always_inline)) {
     if (wave == 0) lstat[buf][0][lane] = -x * kLog2eB;
-    else if (wave == 1) lstat[buf][1][lane] = x;
+    else if (wave == 1) lstat[buf][1][lane] = -x;
   };
   float st = 0.0f;
   if (nt > 0) {
@@ -467,7 +467,16 @@ __global__ __launch_bounds__(256, D == 128 ? 1 : 2) void swa_bf16_dkdv_kernel(Sw
 #pragma unroll
       for (int qb = 0; qb < 2; ++qb) {
         // S and dP for queries r0 + 32 qb + crow(v, h) (rows) and key k0 + kc (column).
-        v16f s = v16f{}, dp = v16f{};
+        // dP starts at -Delta (rows crow(4 i + e, h) = 8 i + 4 h + e: four consecutive stats per i),
+        // so the products leave dP - Delta and the softmax saves a subtraction a score: with the dQ
+        // kernel's, backward 566 -> 552 us at B2 H20 T8192 D64 W2048.
+        v16f s = v16f{}, dp;
+        const float4* dl4 = reinterpret_cast<const float4*>(&lstat[buf][1][32 * qb + 4 * h]);
+#pragma unroll
+        for (int i = 0; i < 4; ++i) {
+          const float4 dl = dl4[2 * i];
+          dp[4 * i] = dl.x; dp[4 * i + 1] = dl.y; dp[4 * i + 2] = dl.z; dp[4 * i + 3] = dl.w;
+        }
 #pragma unroll
         for (int ks = 0; ks < KS; ++ks) {
           s = mfma16(nat_frag<D>(lq[buf], qb, ks, lane), kf[ks], s);
@@ -479,19 +488,17 @@ __global__ __launch_bounds__(256, D == 128 ? 1 : 2) void swa_bf16_dkdv_kernel(Sw
           for (int v = 0; v < 16; ++v)
             if ((unsigned)(q0b + crow(v, h) - key) >= (unsigned)W) s[v] = -INFINITY;
         }
-        // Rows crow(4 i + e, h) = 8 i + 4 h + e: four consecutive stats per i.
         const float4* nl4 = reinterpret_cast<const float4*>(&lstat[buf][0][32 * qb + 4 * h]);
-        const float4* dl4 = reinterpret_cast<const float4*>(&lstat[buf][1][32 * qb + 4 * h]);
 #pragma unroll
         for (int i = 0; i < 4; ++i) {
-          const float4 nl = nl4[2 * i], dl = dl4[2 * i];
-          const float nla[4] = {nl.x, nl.y, nl.z, nl.w}, dla[4] = {dl.x, dl.y, dl.z, dl.w};
+          const float4 nl = nl4[2 * i];
+          const float nla[4] = {nl.x, nl.y, nl.z, nl.w};
 #pragma unroll
           for (int e = 0; e < 4; ++e) {
             const int v = 4 * i + e;
             const float pr = __builtin_amdgcn_exp2f(fmaf(s[v], c, nla[e]));
             s[v] = pr;
-            dp[v] = pr * (dp[v] - dla[e]);           // dS / sm_scale
+            dp[v] *= pr;                             // dS / sm_scale
           }
         }
         // dV += P^T dO, dK += dS^T Q: A = this lane's key row, K = the 32 queries of block qb.
@@ -551,6 +558,9 @@ __global__ __launch_bounds__(256, D == 128 ? 1 : 3) void swa_bf16_dq_kernel(SwaB
     qf[ks] = row_frag<D>(p.q + slice, qi, T, ks, lane);
     df[ks] = row_frag<D>(p.dout + o_base(p, bh, D), qi, T, ks, lane, o_ld(p, D));
   }
+  v16f dl0;                                       // the dP products' start: -Delta of the lane's query
+#pragma unroll
+  for (int v = 0; v < 16; ++v) dl0[v] = -dl;
   v16f dq[NDB];
 #pragma unroll
   for (int db = 0; db < NDB; ++db) dq[db] = v16f{};
@@ -583,7 +593,7 @@ __global__ __launch_bounds__(256, D == 128 ? 1 : 3) void swa_bf16_dq_kernel(SwaB
       const int n0 = lo + 64 * j;
 #pragma unroll
       for (int b = 0; b < 2; ++b) {
-        v16f s = v16f{}, dp = v16f{};
+        v16f s = v16f{}, dp = dl0;
 #pragma unroll
         for (int ks = 0; ks < KS; ++ks) {
           s = mfma16(nat_frag<D>(lk[buf], b, ks, lane), qf[ks], s);
@@ -600,7 +610,7 @@ __global__ __launch_bounds__(256, D == 128 ? 1 : 3) void swa_bf16_dq_kernel(SwaB
 #pragma unroll
         for (int v = 0; v < 16; ++v) {
           const float pr = __builtin_amdgcn_exp2f(fmaf(s[v], c, nlse2));
-          dp[v] = pr * (dp[v] - dl);                  // dS / sm_scale
+          dp[v] *= pr;                                // dS / sm_scale
         }
         // dQ^T += K^T dS^T: A = K^T (dims as rows, keys of block b as K), B = dS^T (this lane's query).
 #pragma unroll
