@@ -464,8 +464,20 @@ __global__ __launch_bounds__(256, D == 128 ? 1 : 2) void swa_bf16_dkdv_kernel(Sw
     }
     if (j >= ta && j <= tb) {
       const int r0 = lo + 64 * j;                    // first query of the tile
+      // One wave a SIMD at D = 128: nothing else covers the fragment reads' latency, so a block's
+      // fragments are read before its products, those of dV / dK before the softmax (backward 327
+      // -> 291 us at B2 H16 T4096 W1024). With more waves it changes nothing (D 64) or costs them.
+      constexpr bool AHEAD = D == 128;
+      v8bf fq[AHEAD ? KS : 1], fo[AHEAD ? KS : 1], tq_[2][AHEAD ? NDB : 1], tdo_[2][AHEAD ? NDB : 1];
 #pragma unroll
       for (int qb = 0; qb < 2; ++qb) {
+        if constexpr (AHEAD) {
+#pragma unroll
+          for (int ks = 0; ks < KS; ++ks) {
+            fq[ks] = nat_frag<D>(lq[buf], qb, ks, lane);
+            fo[ks] = nat_frag<D>(ldo[buf], qb, ks, lane);
+          }
+        }
         // S and dP for queries r0 + 32 qb + crow(v, h) (rows) and key k0 + kc (column).
         // dP starts at -Delta (rows crow(4 i + e, h) = 8 i + 4 h + e: four consecutive stats per i),
         // so the products leave dP - Delta and the softmax saves a subtraction a score: with the dQ
@@ -477,10 +489,25 @@ __global__ __launch_bounds__(256, D == 128 ? 1 : 2) void swa_bf16_dkdv_kernel(Sw
           const float4 dl = dl4[2 * i];
           dp[4 * i] = dl.x; dp[4 * i + 1] = dl.y; dp[4 * i + 2] = dl.z; dp[4 * i + 3] = dl.w;
         }
+        if constexpr (AHEAD) {
 #pragma unroll
-        for (int ks = 0; ks < KS; ++ks) {
-          s = mfma16(nat_frag<D>(lq[buf], qb, ks, lane), kf[ks], s);
-          dp = mfma16(nat_frag<D>(ldo[buf], qb, ks, lane), vf[ks], dp);
+          for (int ks = 0; ks < KS; ++ks) {
+            s = mfma16(fq[ks], kf[ks], s);
+            dp = mfma16(fo[ks], vf[ks], dp);
+          }
+#pragma unroll
+          for (int hs = 0; hs < 2; ++hs)
+#pragma unroll
+            for (int db = 0; db < NDB; ++db) {
+              tdo_[hs][db] = trr_frag<D>(ldo[buf], db, 2 * qb + hs, lane);
+              tq_[hs][db] = trr_frag<D>(lq[buf], db, 2 * qb + hs, lane);
+            }
+        } else {
+#pragma unroll
+          for (int ks = 0; ks < KS; ++ks) {
+            s = mfma16(nat_frag<D>(lq[buf], qb, ks, lane), kf[ks], s);
+            dp = mfma16(nat_frag<D>(ldo[buf], qb, ks, lane), vf[ks], dp);
+          }
         }
         const int q0b = r0 + 32 * qb;
         if (!(q0b >= k0 + 31 && q0b + 31 - k0 < W)) {
@@ -507,8 +534,8 @@ __global__ __launch_bounds__(256, D == 128 ? 1 : 2) void swa_bf16_dkdv_kernel(Sw
           const v8bf pa = pack_frag(s, hs), da = pack_frag(dp, hs);
 #pragma unroll
           for (int db = 0; db < NDB; ++db) {
-            dv[db] = mfma16(pa, trr_frag<D>(ldo[buf], db, 2 * qb + hs, lane), dv[db]);
-            dk[db] = mfma16(da, trr_frag<D>(lq[buf], db, 2 * qb + hs, lane), dk[db]);
+            dv[db] = mfma16(pa, AHEAD ? tdo_[hs][db] : trr_frag<D>(ldo[buf], db, 2 * qb + hs, lane), dv[db]);
+            dk[db] = mfma16(da, AHEAD ? tq_[hs][db] : trr_frag<D>(lq[buf], db, 2 * qb + hs, lane), dk[db]);
           }
         }
       }
