@@ -54,14 +54,16 @@ struct SwaB16Params {
   const uint16_t* v;
   const uint16_t* o;      // forward output (backward: read)
   const uint16_t* dout;   // backward only
-  uint16_t* out;          // forward: O; dq kernel: dQ
-  uint16_t* out2;         // dkdv kernel: dK
-  uint16_t* out3;         // dkdv kernel: dV
+  uint16_t* out;          // forward: O; backward: dQ
+  uint16_t* out2;         // backward: dK
+  uint16_t* out3;         // backward: dV
   float* lse;             // [B, H, T]
   float* delta;           // [B, H, T]
   int H, T, W, nblk, nwg; // nblk: 128-row blocks per (b, h)
-  int ramp;               // blocks per slice whose band is cut short by the sequence's start / end
+  int ramp;               // query blocks per slice whose band is cut short by the sequence's start
+  int ramp_k;             // key blocks per slice whose band is cut short by its end
   int group_slices;       // slices per dispatch group (one XCD's share when it is whole slices)
+  int wg0;                // backward kernel: the launch's first workgroup, of 2 nwg
   float sm_scale;
   int64_t rows;           // B * H * T (delta kernel)
   int o_tmaj;             // O and dO token-major, (B, T, H, D): rows of a (b, h) slice H D apart
@@ -203,20 +205,19 @@ __device__ __forceinline__ void wait_all_loads() {
 // XCD-contiguous work numbering (as in the FP8 kernel).
 // Contiguous work per XCD when the slices split evenly over the 8 XCDs; otherwise round-robin
 // over the XCDs, so each XCD gets an even share of the long and short work items.
-__device__ __forceinline__ int xcd_id(const SwaB16Params& p) {
-  int L = (int)blockIdx.x;
+__device__ __forceinline__ int xcd_id(const SwaB16Params& p, int L) {
   if (p.group_slices * 8 * p.nblk == p.nwg) L = (L & 7) * (p.nwg >> 3) + (L >> 3);
   return L;
 }
 
-// (slice, 128-row block) of this workgroup. Inside one XCD's group of slices the blocks with a
+// (slice, 128-row block) of workgroup L. Inside one XCD's group of slices the blocks with a
 // full-length band come first, slice by slice (consecutive blocks share K / V or Q / dO tiles in
 // that XCD's L2), then the `ramp` short-band blocks in decreasing band length, so the short work
 // items fill the grid's drain. Query-block kernels: the short blocks are a slice's first ones (their
 // band starts at key 0); the key-block kernel: its last ones (their band ends at query T - 1).
-__device__ __forceinline__ void band_order(const SwaB16Params& p, bool ramp_at_end, int& bh, int& blk) {
-  const int L = xcd_id(p);
-  const int gs = p.group_slices, R = p.ramp, nfull = p.nblk - R;
+__device__ __forceinline__ void band_order(const SwaB16Params& p, int wg, bool ramp_at_end, int& bh, int& blk) {
+  const int L = xcd_id(p, wg);
+  const int gs = p.group_slices, R = ramp_at_end ? p.ramp_k : p.ramp, nfull = p.nblk - R;
   const int gi = L / (gs * p.nblk), i = L % (gs * p.nblk);
   if (i < gs * nfull) {
     bh = gi * gs + i / nfull;
@@ -239,7 +240,7 @@ __global__ __launch_bounds__(256, 2) void swa_bf16_fwd_kernel(SwaB16Params p) {
   __shared__ __align__(16) uint8_t lv[2][NAT];
   const int tid = threadIdx.x, lane = tid & 63, wave = __builtin_amdgcn_readfirstlane(tid >> 6), h = lane >> 5, qc = lane & 31;
   int bh, mt;
-  band_order(p, false, bh, mt);
+  band_order(p, (int)blockIdx.x, false, bh, mt);
   const int T = p.T, W = p.W;
   const int m0 = mt * 128, q0 = m0 + 32 * wave;
   const int64_t slice = (int64_t)bh * T * D;
@@ -388,14 +389,17 @@ __global__ __launch_bounds__(256) void swa_bf16_delta_kernel(SwaB16Params p) {
 // ---------------------------------------------------------------- backward: dK, dV
 
 template <int D>
-__global__ __launch_bounds__(256, D == 128 ? 1 : 2) void swa_bf16_dkdv_kernel(SwaB16Params p) {
-  constexpr int KS = D / 16, NDB = D / 32, NAT = 64 * D * 2;
-  __shared__ __align__(16) uint8_t lq[2][NAT];     // Q tile: A operand of S, read transposed for dK
-  __shared__ __align__(16) uint8_t ldo[2][NAT];    // dO tile: A operand of dP, read transposed for dV
-  __shared__ __align__(16) float lstat[2][2][64];  // -L log2(e) and -Delta of the tile's queries
+using TilePair = uint8_t[2][64 * D * 2];          // two buffers of a 64-row tile
+
+// lq: Q tile, A operand of S, read transposed for dK; ldo: dO tile, A operand of dP, read transposed
+// for dV; lstat: -L log2(e) and -Delta of the tile's queries.
+template <int D>
+__device__ __forceinline__ void dkdv_block(const SwaB16Params& p, int wg, TilePair<D>& lq, TilePair<D>& ldo,
+                                           float (&lstat)[2][2][64]) {
+  constexpr int KS = D / 16, NDB = D / 32;
   const int tid = threadIdx.x, lane = tid & 63, wave = __builtin_amdgcn_readfirstlane(tid >> 6), h = lane >> 5, kc = lane & 31;
   int bh, nt0;
-  band_order(p, true, bh, nt0);
+  band_order(p, wg, true, bh, nt0);
   const int T = p.T, W = p.W;
   const int k0w = nt0 * 128, k0 = k0w + 32 * wave;     // this wave's 32 keys
   const int64_t slice = (int64_t)bh * T * D;
@@ -561,14 +565,13 @@ __global__ __launch_bounds__(256, D == 128 ? 1 : 2) void swa_bf16_dkdv_kernel(Sw
 
 // ---------------------------------------------------------------- backward: dQ
 
+// lk: K tile, A operand of S^T, read transposed for dQ^T; lv: V tile, natural (A operand of dP^T).
 template <int D>
-__global__ __launch_bounds__(256, D == 128 ? 1 : 3) void swa_bf16_dq_kernel(SwaB16Params p) {
-  constexpr int KS = D / 16, NDB = D / 32, NAT = 64 * D * 2;
-  __shared__ __align__(16) uint8_t lk[2][NAT];     // K tile: A operand of S^T, read transposed for dQ^T
-  __shared__ __align__(16) uint8_t lv[2][NAT];     // V tile, natural (A operand of dP^T)
+__device__ __forceinline__ void dq_block(const SwaB16Params& p, int wg, TilePair<D>& lk, TilePair<D>& lv) {
+  constexpr int KS = D / 16, NDB = D / 32;
   const int tid = threadIdx.x, lane = tid & 63, wave = __builtin_amdgcn_readfirstlane(tid >> 6), h = lane >> 5, qc = lane & 31;
   int bh, mt;
-  band_order(p, false, bh, mt);
+  band_order(p, wg, false, bh, mt);
   const int T = p.T, W = p.W;
   const int m0 = mt * 128, q0 = m0 + 32 * wave;
   const int64_t slice = (int64_t)bh * T * D;
@@ -665,6 +668,58 @@ __global__ __launch_bounds__(256, D == 128 ? 1 : 3) void swa_bf16_dq_kernel(SwaB
         *reinterpret_cast<uint2*>(op + d) = w;
       }
   }
+}
+
+// ---------------------------------------------------------------- backward kernels
+
+// dK / dV and dQ in one launch: workgroups 0 .. nwg - 1 are the dK / dV blocks (the longer ones, so
+// they start first), the next nwg the dQ blocks. Neither needs the other, and one after the other
+// each left compute units idle: small grids all the time (96 workgroups each at T = 1500, 8 heads),
+// large ones while the last blocks drain. Backward (Delta included), two launches -> one, us:
+// D = 64: B1 H8 T1500 W500 33.6 -> 23.4, B1 H20 T4096 W2048 143 -> 131, B2 H20 T8192 W2048 552 -> 520;
+// D = 32: B1 H8 T1500 W500 26.0 -> 16.7; D = 128: B1 H8 T1500 W500 50.4 -> 31.8. The same bits.
+// The tiles' LDS: one array at D = 32 and 64, which the register allocator takes 166 VGPRs for at
+// D = 64, three waves a SIMD (as two arrays 176, two waves: 553 us at T8192), two at D = 128, where
+// one wave runs either way (one array: 33 us at T1500, 1251 against 1215 at B2 H20 T8192 W2048).
+template <int D>
+__global__ __launch_bounds__(256, D == 128 ? 1 : 2) void swa_bf16_bwd_kernel(SwaB16Params p) {
+  __shared__ __align__(16) TilePair<D> t[D == 128 ? 1 : 2];
+  __shared__ __align__(16) float stat[2][2][64];
+  auto run = [&](TilePair<D>& a, TilePair<D>& b) __attribute__((always_inline)) {
+    const int wg = p.wg0 + (int)blockIdx.x;
+    if (wg < p.nwg) dkdv_block<D>(p, wg, a, b, stat);
+    else dq_block<D>(p, wg - p.nwg, a, b);
+  };
+  if constexpr (D == 128) {
+    __shared__ __align__(16) TilePair<D> t1;
+    run(t[0], t1);
+  } else {
+    run(t[0], t[1]);
+  }
+}
+
+// The two as launches of their own, at D = 128 and large grids: there dQ alone fits two waves a SIMD
+// (224 VGPRs), beside dK / dV one.
+__global__ __launch_bounds__(256, 1) void swa_bf16_dkdv128_kernel(SwaB16Params p) {
+  __shared__ __align__(16) TilePair<128> lq;
+  __shared__ __align__(16) TilePair<128> ldo;
+  __shared__ __align__(16) float lstat[2][2][64];
+  dkdv_block<128>(p, (int)blockIdx.x, lq, ldo, lstat);
+}
+__global__ __launch_bounds__(256, 1) void swa_bf16_dq128_kernel(SwaB16Params p) {
+  __shared__ __align__(16) TilePair<128> lk;
+  __shared__ __align__(16) TilePair<128> lv;
+  dq_block<128>(p, (int)blockIdx.x, lk, lv);
+}
+
+// One launch for both: at D = 32 and 64 always, as they lose no wave by it (but a grid is less than
+// 2^32 threads, which one of many short slices comes near). At D = 128 while the
+// workgroups of both are at most two rounds of the compute units (one workgroup each): 0.62-0.64 of
+// the two launches' time up to one round, 0.90 at two (B2 H16 T1024 W512: 54.8 -> 49.6 us). Beyond, the
+// lost dQ wave and the shorter drain decide by shape: 0.92 at B2 H16 T2048, 0.98 at B2 H16 T4096, 1.02-
+// 1.04 at B1 H8 T8192 W256, B3 H12 T3000 W777 and B2 H20 T8192 W2048, so those keep two launches.
+static bool one_launch(int64_t D, int64_t nwg) {
+  return D != 128 ? 2 * nwg < (1ll << 32) / 256 : 2 * nwg <= 2 * (int64_t)compute_units();
 }
 
 // ---------------------------------------------------------------- host
@@ -775,27 +830,28 @@ static int swa_bf16_bwd(const void* q, const void* k, const void* v, const void*
   p.rows = B * H * T;
   const int64_t threads = p.rows * (D / 8);
   const dim3 dgrid((unsigned)((threads + 255) / 256));
-  const dim3 grid((unsigned)p.nwg);
   p.group_slices = group_slices(B * H, p.nwg);
-  SwaB16Params pk = p;
-  pk.out2 = static_cast<uint16_t*>(dk); pk.out3 = static_cast<uint16_t*>(dv);
-  pk.ramp = key_ramp(p);
-  SwaB16Params pq = p;
-  pq.out = static_cast<uint16_t*>(dq);
-  pq.ramp = query_ramp(p);
+  p.out = static_cast<uint16_t*>(dq); p.out2 = static_cast<uint16_t*>(dk); p.out3 = static_cast<uint16_t*>(dv);
+  p.ramp = query_ramp(p);
+  p.ramp_k = key_ramp(p);
   const void* kd = D == 32 ? reinterpret_cast<const void*>(&swa_bf16_delta_kernel<32>)
                  : D == 64 ? reinterpret_cast<const void*>(&swa_bf16_delta_kernel<64>)
                            : reinterpret_cast<const void*>(&swa_bf16_delta_kernel<128>);
-  const void* kk = D == 32 ? reinterpret_cast<const void*>(&swa_bf16_dkdv_kernel<32>)
-                 : D == 64 ? reinterpret_cast<const void*>(&swa_bf16_dkdv_kernel<64>)
-                           : reinterpret_cast<const void*>(&swa_bf16_dkdv_kernel<128>);
-  const void* kq = D == 32 ? reinterpret_cast<const void*>(&swa_bf16_dq_kernel<32>)
-                 : D == 64 ? reinterpret_cast<const void*>(&swa_bf16_dq_kernel<64>)
-                           : reinterpret_cast<const void*>(&swa_bf16_dq_kernel<128>);
-  const Timer tm = take_timer();   // start on the delta kernel, stop on the dQ kernel
+  const void* kb = D == 32 ? reinterpret_cast<const void*>(&swa_bf16_bwd_kernel<32>)
+                 : D == 64 ? reinterpret_cast<const void*>(&swa_bf16_bwd_kernel<64>)
+                           : reinterpret_cast<const void*>(&swa_bf16_bwd_kernel<128>);
+  const Timer tm = take_timer();   // start on the delta kernel, stop on the last kernel
   (void)launch_ext(kd, dgrid, dim3(256), 0, s, p, tm.start, nullptr);
-  (void)launch_ext(kk, grid, dim3(256), 0, s, pk, nullptr, nullptr);
-  (void)launch_ext(kq, grid, dim3(256), 0, s, pq, nullptr, tm.stop);
+  if (one_launch(D, p.nwg)) {
+    (void)launch_ext(kb, dim3((unsigned)(2 * p.nwg)), dim3(256), 0, s, p, nullptr, tm.stop);
+  } else if (const dim3 grid((unsigned)p.nwg); D != 128) {
+    (void)launch_ext(kb, grid, dim3(256), 0, s, p, nullptr, nullptr);
+    p.wg0 = p.nwg;
+    (void)launch_ext(kb, grid, dim3(256), 0, s, p, nullptr, tm.stop);
+  } else {
+    (void)launch_ext(reinterpret_cast<const void*>(&swa_bf16_dkdv128_kernel), grid, dim3(256), 0, s, p, nullptr, nullptr);
+    (void)launch_ext(reinterpret_cast<const void*>(&swa_bf16_dq128_kernel), grid, dim3(256), 0, s, p, nullptr, tm.stop);
+  }
   return check_launch(name);
 }
 
