@@ -61,11 +61,8 @@ struct QuantParams {
   QTensor t[3];
   int64_t d0, d1, d2, d3;      // B, H, T, D
   int64_t nchunks;             // chunks per slice
-  int64_t part_stride;         // partials per tensor
-  int64_t fold_n, fold_run;    // partials of a scale group, in runs of fold_run (d1 nchunks apart)
   uint32_t* partials;          // [tensor][d0*d1][nchunks] |x| max bit patterns
   int granularity;
-  int64_t groups;              // scale groups per tensor
   const uint32_t* amax_given;  // optional [tensor][groups] |x| max bit patterns (no amax pass)
 };
 
@@ -80,21 +77,12 @@ __device__ __forceinline__ uint32_t block_max_u32(uint32_t m, uint32_t* lds4) {
   return r;
 }
 
-// (v / vpr, v % vpr), the row and column of the 16-byte vector v of a chunk: a shift where vpr is a
-// power of two (uniform over the launch), a 32-bit division below 2^32.
-struct VecPos { int64_t row, col; };
-__device__ __forceinline__ VecPos vec_pos(int64_t v, int64_t vpr) {
-  if ((vpr & (vpr - 1)) == 0) return {v >> (63 - __builtin_clzll(vpr)), v & (vpr - 1)};
-  if (((v | vpr) >> 32) == 0) return {(int64_t)((uint32_t)v / (uint32_t)vpr), (int64_t)((uint32_t)v % (uint32_t)vpr)};
-  return {v / vpr, v % vpr};
-}
-
 // Element offset of the 16-byte vector v of chunk rows [r0, ...) inside a slice.
 __device__ __forceinline__ int64_t vec_offset(const QTensor& t, int64_t r0, int64_t v, int64_t vpr,
                                               int n, int64_t d3) {
   if (t.rows_packed) return r0 * d3 + v * n;
-  const VecPos pos = vec_pos(v, vpr);
-  return (r0 + pos.row) * t.s2 + pos.col * n;
+  const int64_t row = r0 + v / vpr, cv = v % vpr;
+  return row * t.s2 + cv * n;
 }
 
 // The pre-attention transform of CausalSelfAttention.qkv_heads on one 16-byte vector (column
@@ -121,9 +109,7 @@ __global__ __launch_bounds__(kThreads) void amax_kernel(QuantParams p) {
   __shared__ uint32_t red[kThreads / 64];
   const QTensor& t = p.t[blockIdx.z];
   const int64_t slice = blockIdx.y;
-  asm volatile("" ::"s"(t.x), "s"(t.s0), "s"(t.s1), "s"(t.s2), "s"(t.rows_packed), "s"(p.d1), "s"(p.d2), "s"(p.d3),
-               "s"(p.nchunks), "s"(p.part_stride), "s"(p.partials));     // loaded at once: see quant_kernel
-  const uint32_t i0 = blockIdx.y / (uint32_t)p.d1, i1 = blockIdx.y % (uint32_t)p.d1;
+  const int64_t i0 = slice / p.d1, i1 = slice % p.d1;
   const int64_t r0 = (int64_t)blockIdx.x * kRowsPerChunk;
   const int64_t r1 = min(p.d2, r0 + kRowsPerChunk);
   const T* base = static_cast<const T*>(t.x) + i0 * t.s0 + i1 * t.s1;
@@ -147,8 +133,7 @@ __global__ __launch_bounds__(kThreads) void amax_kernel(QuantParams p) {
 #pragma unroll
       for (int u = 0; u < U; ++u) {
         const int64_t v = v0 + (int64_t)u * kThreads;
-        const VecPos pos = vec_pos(v, vpr);
-        qk_transform<T>(t, f[u], r0 + pos.row, pos.col, (int)vpr, p.d3, v < nvec);
+        qk_transform<T>(t, f[u], r0 + v / vpr, v % vpr, (int)vpr, p.d3, v < nvec);
       }
     }
 #pragma unroll
@@ -158,28 +143,41 @@ __global__ __launch_bounds__(kThreads) void amax_kernel(QuantParams p) {
   }
   m = block_max_u32(m, red);
   if (threadIdx.x == 0)
-    p.partials[blockIdx.z * p.part_stride + slice * p.nchunks + blockIdx.x] = m;
+    p.partials[((int64_t)blockIdx.z * p.d0 * p.d1 + slice) * p.nchunks + blockIdx.x] = m;
 }
 
-// Fold the partials of the scale group `group` of one tensor: fold_n of them in runs of fold_run.
-__device__ __forceinline__ uint32_t group_amax(const QuantParams& p, const uint32_t* part, int64_t group,
-                                               uint32_t* red) {
+// Fold the partials of this workgroup's scale group.
+__device__ __forceinline__ uint32_t group_amax(const QuantParams& p, const uint32_t* part,
+                                               int64_t slice, int64_t i1, uint32_t* red) {
   uint32_t m = 0;
-  part += group * p.nchunks;
-  for (int64_t i = threadIdx.x; i < p.fold_n; i += kThreads) {
-    int64_t o = i;
-    if (p.fold_n != p.fold_run) {
-      const VecPos pos = vec_pos(i, p.fold_run);
-      o = pos.row * p.d1 * p.nchunks + pos.col;
+  if (p.granularity == FLW_SCALE_TENSOR) {
+    const int64_t n = p.d0 * p.d1 * p.nchunks;
+    for (int64_t i = threadIdx.x; i < n; i += kThreads) { uint32_t a = part[i]; m = m > a ? m : a; }
+  } else if (p.granularity == FLW_SCALE_HEAD) {
+    const int64_t n = p.d0 * p.nchunks;
+    for (int64_t i = threadIdx.x; i < n; i += kThreads) {
+      const int64_t b = i / p.nchunks, c = i % p.nchunks;
+      uint32_t a = part[(b * p.d1 + i1) * p.nchunks + c];
+      m = m > a ? m : a;
     }
-    const uint32_t a = part[o];
-    m = m > a ? m : a;
+  } else {
+    for (int64_t i = threadIdx.x; i < p.nchunks; i += kThreads) {
+      uint32_t a = part[slice * p.nchunks + i];
+      m = m > a ? m : a;
+    }
   }
   return block_max_u32(m, red);
 }
 
 __device__ __forceinline__ int64_t group_index(int gran, int64_t slice, int64_t i1) {
   return gran == FLW_SCALE_TENSOR ? 0 : (gran == FLW_SCALE_HEAD ? i1 : slice);
+}
+
+__device__ __forceinline__ bool writes_scale(int gran, int64_t slice, int64_t i0) {
+  if (blockIdx.x != 0 || threadIdx.x != 0) return false;
+  if (gran == FLW_SCALE_TENSOR) return slice == 0;
+  if (gran == FLW_SCALE_HEAD) return i0 == 0;
+  return true;
 }
 
 __device__ __forceinline__ float clamp448(float y) {
@@ -227,20 +225,13 @@ __global__ __launch_bounds__(kThreads) void quant_kernel(QuantParams p) {
   const int64_t slice = (int64_t)(gridDim.y - 1 - blockIdx.y);
   const int64_t bx = (int64_t)(gridDim.x - 1 - blockIdx.x);
   const QTensor& t = p.t[zi];
-  // Every argument the workgroup needs is loaded here at once: read where they are used they are a
-  // chain of scalar-cache misses in front of every load, and with 64-bit divisions in place of
-  // vec_pos they were the difference at small launches and ragged ones (amax + quantise pass,
-  // D = 64: [1, 8, 1024] 10.2 -> 9.5 us, [1, 20, 4096] 18.2 -> 16.6, D = 128 [2, 8, 3001] 20.8 -> 19.8,
-  // [4, 16, 4096] 37.0 -> 36.4). Reading the first vectors before the fold, 1024-thread workgroups,
-  // and one pass whose workgroups each read their whole scale group were all no faster or slower.
-  asm volatile("" ::"s"(t.x), "s"(t.s0), "s"(t.s1), "s"(t.s2), "s"(t.out8), "s"(t.outx), "s"(t.scale_out),
-               "s"(t.layout), "s"(t.rows_packed), "s"(t.defer), "s"(t.rcp_out), "s"(p.d1), "s"(p.d2), "s"(p.d3),
-               "s"(p.nchunks), "s"(p.part_stride), "s"(p.fold_n), "s"(p.fold_run), "s"(p.partials),
-               "s"(p.granularity), "s"(p.groups), "s"(p.amax_given));
-  const uint32_t i0 = (uint32_t)slice / (uint32_t)p.d1, i1 = (uint32_t)slice % (uint32_t)p.d1;
-  const int64_t group = group_index(p.granularity, slice, i1);
-  const float amax = __uint_as_float(
-      p.amax_given ? p.amax_given[zi * p.groups + group] : group_amax(p, p.partials + zi * p.part_stride, group, red));
+  const int64_t i0 = slice / p.d1, i1 = slice % p.d1;
+  const uint32_t* part = p.partials + (int64_t)zi * p.d0 * p.d1 * p.nchunks;
+
+  const int64_t ngroups = p.granularity == FLW_SCALE_TENSOR ? 1 : (p.granularity == FLW_SCALE_HEAD ? p.d1 : p.d0 * p.d1);
+  const float amax = p.amax_given
+      ? __uint_as_float(p.amax_given[zi * ngroups + group_index(p.granularity, slice, i1)])
+      : __uint_as_float(group_amax(p, part, slice, i1, red));
   float scale;
   if (MODE == 1 && kBf16) {
     // base.py:198-199 under bf16: clamp and /448 are bf16 tensor ops
@@ -251,9 +242,9 @@ __global__ __launch_bounds__(kThreads) void quant_kernel(QuantParams p) {
   }
   const bool fast = MODE == 0 && __builtin_isfinite(amax);   // uniform over the workgroup
   const float rcp = 1.0f / scale;                            // IEEE: correctly rounded
-  if (bx == 0 && slice == group && threadIdx.x == 0) {       // the group's first slice, its first chunk
-    t.scale_out[group] = scale;
-    if (MODE == 0 && t.rcp_out != nullptr) t.rcp_out[group] = rcp;
+  if (writes_scale(p.granularity, slice, i0)) {
+    t.scale_out[group_index(p.granularity, slice, i1)] = scale;
+    if (MODE == 0 && t.rcp_out != nullptr) t.rcp_out[group_index(p.granularity, slice, i1)] = rcp;
   }
   if (MODE == 0 && t.defer && fast) return;                  // codes made by the attention kernel
   // A given amax is the caller's claim about the data (a producer's epilogue maximum, or a
@@ -291,8 +282,7 @@ __global__ __launch_bounds__(kThreads) void quant_kernel(QuantParams p) {
 #pragma unroll
       for (int u = 0; u < kUnroll; ++u) {
         const int64_t v = v0 + (int64_t)u * kThreads;
-        const VecPos pos = vec_pos(v, vpr);
-        qk_transform<T>(t, f[u], r0 + pos.row, pos.col, (int)vpr, p.d3, v < nvec);
+        qk_transform<T>(t, f[u], r0 + v / vpr, v % vpr, (int)vpr, p.d3, v < nvec);
         if (t.tout != nullptr && v < nvec) {
           T* dst = static_cast<T*>(t.tout) + (slice * p.d2 + r0) * p.d3 + v * V::N;
           if constexpr (sizeof(T) == 2) {
@@ -327,8 +317,7 @@ __global__ __launch_bounds__(kThreads) void quant_kernel(QuantParams p) {
           else *reinterpret_cast<uint32_t*>(dst) = w[0];
         } else {
           // the chunk's rows staged as they are (vrow_offset), re-read in the tile order below
-          const VecPos pos = vec_pos(v, vpr);
-          const int lrow = (int)pos.row, d = (int)(pos.col * V::N), D = (int)p.d3;
+          const int lrow = (int)(v / vpr), d = (int)((v % vpr) * V::N), D = (int)p.d3;
           uint8_t* dst = tile_lds + (lrow >> 6) * 64 * D + vrow_offset(lrow & 63, d >> 4, D) + (d & 15);
           const bool pad = v >= nvec;
           if (V::N == 8) *reinterpret_cast<uint2*>(dst) = pad ? make_uint2(0, 0) : make_uint2(w[0], w[1]);
@@ -763,17 +752,6 @@ static size_t partial_bytes(int64_t B, int64_t H, int64_t T) {
   return (size_t)(B * H * nchunks_of(T)) * sizeof(uint32_t);
 }
 
-// The shape, and what the kernels derive from it.
-static void set_shape(QuantParams& p, int64_t B, int64_t H, int64_t T, int64_t D, int granularity) {
-  p.d0 = B; p.d1 = H; p.d2 = T; p.d3 = D;
-  p.nchunks = nchunks_of(T);
-  p.part_stride = B * H * p.nchunks;
-  p.granularity = granularity;
-  p.groups = granularity == FLW_SCALE_TENSOR ? 1 : granularity == FLW_SCALE_HEAD ? H : B * H;
-  p.fold_n = p.part_stride / p.groups;
-  p.fold_run = granularity == FLW_SCALE_HEAD ? p.nchunks : p.fold_n;
-}
-
 template <int MODE>
 static int launch_quant(const QuantParams& p, int ntensors, int dtype, hipStream_t s, const char* name,
                         Timer tm) {
@@ -847,8 +825,8 @@ int quant_bhtd_n(int n, const void* const* xs, int dtype, int64_t B, int64_t H, 
     p.t[0].defer = 1;
     p.t[0].rcp_out = q_rcp_deferred;
   }
-  set_shape(p, B, H, T, D, granularity);
-  p.partials = static_cast<uint32_t*>(ws);
+  p.d0 = B; p.d1 = H; p.d2 = T; p.d3 = D;
+  p.nchunks = nchunks_of(T); p.partials = static_cast<uint32_t*>(ws); p.granularity = granularity;
   p.amax_given = amax_given;
   return launch_quant<0>(p, n, dtype, stream, "flw_quant_e4m3", tm);
 }
@@ -864,8 +842,11 @@ int quant_bhtd(const void* x, int dtype, int64_t B, int64_t H, int64_t T, int64_
 // One workgroup per scale group (grid.x) folds that group's amax partials into amax_out.
 __global__ __launch_bounds__(kThreads) void amax_fold_kernel(QuantParams p, uint32_t* __restrict__ amax_out) {
   __shared__ uint32_t red[kThreads / 64];
-  const uint32_t m = group_amax(p, p.partials, blockIdx.x, red);
-  if (threadIdx.x == 0) amax_out[blockIdx.x] = m;
+  const int64_t g = blockIdx.x;
+  const int64_t slice = p.granularity == FLW_SCALE_BH ? g : 0;
+  const int64_t i1 = p.granularity == FLW_SCALE_HEAD ? g : slice % p.d1;
+  const uint32_t m = group_amax(p, p.partials, slice, i1, red);
+  if (threadIdx.x == 0) amax_out[g] = m;
 }
 
 // The amax pass alone: |x| max per scale group, as the bit patterns of non-negative fp32 values.
@@ -880,14 +861,15 @@ int amax_bhtd(const void* x, int dtype, int64_t B, int64_t H, int64_t T, int64_t
               partial_bytes(B, H, T));
   QuantParams p{};
   set_tensor(p.t[0], x, sb, sh, st, D, FLW_LAYOUT_BHTD, nullptr, nullptr, nullptr);
-  set_shape(p, B, H, T, D, granularity);
-  p.partials = static_cast<uint32_t*>(ws);
+  p.d0 = B; p.d1 = H; p.d2 = T; p.d3 = D;
+  p.nchunks = nchunks_of(T); p.partials = static_cast<uint32_t*>(ws); p.granularity = granularity;
+  const int64_t G = granularity == FLW_SCALE_TENSOR ? 1 : (granularity == FLW_SCALE_HEAD ? H : B * H);
   const void* ka = dtype == FLW_F32 ? reinterpret_cast<const void*>(&amax_kernel<float>)
                                     : reinterpret_cast<const void*>(&amax_kernel<uint16_t>);
   const Timer tm = take_timer();
   (void)launch_ext(ka, dim3((unsigned)p.nchunks, (unsigned)(B * H), 1u), dim3(kThreads), 0, stream, p,
                    tm.start, nullptr);
-  (void)launch_args(reinterpret_cast<const void*>(&amax_fold_kernel), dim3((unsigned)p.groups), dim3(kThreads), 0,
+  (void)launch_args(reinterpret_cast<const void*>(&amax_fold_kernel), dim3((unsigned)G), dim3(kThreads), 0,
                     stream, nullptr, tm.stop, p, amax_out);
   return check_launch("flw_amax_e4m3");
 }
@@ -1007,8 +989,8 @@ extern "C" int flw_fake_quant_e4m3(const void* x, int dtype, int64_t B, int64_t 
     sc = reinterpret_cast<float*>(static_cast<uint8_t*>(workspace) + partial_bytes(B, H, T));
   }
   set_tensor(p.t[0], x, stride_b, stride_h, stride_t, D, FLW_LAYOUT_BHTD, nullptr, out, sc);
-  set_shape(p, B, H, T, D, granularity);
-  p.partials = static_cast<uint32_t*>(workspace);
+  p.d0 = B; p.d1 = H; p.d2 = T; p.d3 = D;
+  p.nchunks = nchunks_of(T); p.partials = static_cast<uint32_t*>(workspace); p.granularity = granularity;
   return launch_quant<1>(p, 1, dtype, static_cast<hipStream_t>(stream), "flw_fake_quant_e4m3", take_timer());
 }
 
@@ -1262,9 +1244,11 @@ extern "C" int flw_quant_tensor_t_e4m3(const void* x, int64_t rows, int64_t cols
   const int64_t d2 = flat ? rows * cols / fc : rows, d3 = flat ? fc : cols;
   set_tensor(p.t[0], x, d2 * (flat ? fc : row_stride), d2 * (flat ? fc : row_stride), flat ? fc : row_stride, d3,
              FLW_LAYOUT_BHTD, nullptr, nullptr, nullptr);
-  set_shape(p, 1, 1, d2, d3, FLW_SCALE_TENSOR);
+  p.d0 = 1; p.d1 = 1; p.d2 = d2; p.d3 = d3;
+  p.nchunks = nchunks_of(d2);
   uint32_t* amax = static_cast<uint32_t*>(workspace);
   p.partials = reinterpret_cast<uint32_t*>(static_cast<uint8_t*>(workspace) + 16);
+  p.granularity = FLW_SCALE_TENSOR;
   FLW_REQUIRE(p.nchunks <= 0x7FFFFFFF, FLW_E_UNSUPPORTED, "matrix too large");
   hipStream_t s = static_cast<hipStream_t>(stream);
   const Timer tm = take_timer();
