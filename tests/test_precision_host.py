@@ -138,3 +138,35 @@ def test_weight_cache_is_a_no_op_without_fp8_layers():
     with fp8_weight_cache(m) as c:
         assert c.entries == []
     assert m[0].forward == before
+
+
+@pytest.mark.parametrize("call", ["scaled_mm", "scaled_mm_plain", "scaled_mm_residual", "transpose_codes",
+                                  "fp8_linear_backward"])
+def test_codes_off_the_gpu_are_refused(call, monkeypatch):
+    """Functions on e4m3 codes refuse CPU tensors before anything is allocated or launched: the native
+    bodies and the raw stream look-up (to which the CPU's device index -1 is the current GPU) are not
+    reached."""
+    from flower_amd import _lib
+    from flower_amd import precision as P
+
+    def reached(*args):
+        raise AssertionError("reached with CPU tensors")
+
+    class Bodies:
+        def __getattr__(self, name):
+            return reached
+
+    monkeypatch.setattr(_lib, "native", Bodies)
+    monkeypatch.setattr(torch._C, "_cuda_getCurrentRawStream", reached, raising=False)
+    a8, b8 = torch.zeros(16, 64, dtype=torch.uint8), torch.zeros(32, 64, dtype=torch.uint8)
+    sa, sb = torch.ones(16), torch.ones(32)
+    with pytest.raises(ValueError, match="Expected a cuda device"):
+        if call == "scaled_mm_residual":
+            P.scaled_mm_residual(a8, sa, b8, sb, torch.zeros(16, 32, dtype=torch.bfloat16))
+        elif call == "transpose_codes":
+            P.transpose_codes(a8)
+        elif call == "fp8_linear_backward":
+            P.fp8_linear_backward(torch.zeros(16, 32, dtype=torch.bfloat16), None, (b8.t().contiguous(), sb[:1]),
+                                  "tensorwise", x_codes=(a8.t().contiguous(), sa[:1]))
+        else:
+            getattr(P, call)(a8, sa, b8, sb)
