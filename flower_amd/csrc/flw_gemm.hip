@@ -1497,30 +1497,26 @@ __global__ __launch_bounds__(256) void fill_u32_kernel(uint32_t* p, int n, uint3
 
 // Compute units of the current device (queried once per device).
 
-// K ranges per output tile a caller's workspace is sized for (flw_fp8_scaled_mm_workspace_bytes):
-// outputs whose 256 x 256 tiles would leave more than half of the compute units idle, each range
-// keeping at least 4 K stages of 128. Whether the GEMM then splits is use_split's decision.
-static int splitk_of(int64_t tiles, int64_t K) {
-  const int cus = compute_units();
-  if (tiles * 2 >= cus) return 1;     // half the GPU or more busy: the finish pass would cost more
-  int sp = (int)(cus / tiles);
-  sp = sp > 8 ? 8 : sp;
-  while (sp > 1 && (K / kFBK) / sp < 4) --sp;
-  return sp < 1 ? 1 : sp;
+// The shapes the tiled kernels take: whole 64-deep K chunks, 32-bit operand offsets. The rest runs on
+// fp8_gemm_kernel.
+static bool tiled(int64_t M, int64_t N, int64_t K) {
+  return K % 64 == 0 && N * K < (1ll << 32) && M * K < (1ll << 32);
+}
+
+// K ranges per 256 x 256 output tile, for the workspace query and the GEMM alike: three where that many
+// fill the GPU and K is long enough to pay for the partials ([3840, 1280] and [3392, 1280] at K = 16384
+// 93 / 90 us against 102 / 99 us unsplit, 61 / 59 against 53 / 52 us at K = 8192), one otherwise. Two
+// ranges, or four and more, measured slower than the smaller tiles unsplit: [4096, 1024] at K = 8192 48
+// -> 37 us, [1024, 1024] at K = 4096 24 -> 10 us.
+static int splitk_of(int64_t M, int64_t N, int64_t K) {
+  const int64_t tiles = ((N + kFBN - 1) / kFBN) * ((M + kFBM - 1) / kFBM);
+  return tiled(M, N, K) && K >= 96 * kFBK && compute_units() / tiles == 3 ? 3 : 1;
 }
 
 static size_t splitk_bytes(int64_t M, int64_t N, int64_t K) {
-  if (K % 64 != 0) return 0;
-  const int64_t tiles = ((N + kFBN - 1) / kFBN) * ((M + kFBM - 1) / kFBM);
-  const int sp = splitk_of(tiles, K);
+  const int sp = splitk_of(M, N, K);
   return sp > 1 ? (size_t)sp * (size_t)M * (size_t)N * sizeof(float) : 0;
 }
-
-// Split over K only where 256 x 256 tiles x 3 ranges fill the GPU and K is long enough to pay for
-// the partials: [3840, 1280] and [3392, 1280] at K = 16384 93 / 90 us against 102 / 99 us unsplit,
-// 61 / 59 against 53 / 52 us at K = 8192. Every other split measured slower than the smaller tiles
-// unsplit: [4096, 1024] at K = 8192 48 -> 37 us, [1024, 1024] at K = 4096 24 -> 10 us.
-static bool use_split(int splits, int64_t K) { return splits == 3 && K >= 96 * kFBK; }
 
 // Output tiles of the FP8 GEMM, n x m. Every one accumulates an output's K products in the same
 // order, so the choice changes the time only.
@@ -1607,19 +1603,18 @@ static int scaled_mm(const uint8_t* x8, int64_t M, int64_t K, const uint8_t* w8,
   p.res = static_cast<const uint16_t*>(res); p.rs = rs;
   FLW_REQUIRE(res == nullptr || (rs >= N && rs % 4 == 0 && ((uintptr_t)res & 7) == 0), FLW_E_INVALID,
               "residual rows must be 8-byte aligned with a stride >= N, a multiple of 4");
-  if (K % 64 == 0 && N * K < (1ll << 32) && M * K < (1ll << 32)) {
+  if (tiled(M, N, K)) {
     const int64_t wide = ((N + kFBN - 1) / kFBN) * ((M + kFBM - 1) / kFBM);
     FLW_REQUIRE(wide <= 0x7FFFFFFF, FLW_E_UNSUPPORTED, "grid too large");
     p.splits = 1;
     p.lds_epi = N % 8 == 0 && ys % 8 == 0 && ((uintptr_t)y & 15) == 0 &&
                 (res == nullptr || (rs % 8 == 0 && ((uintptr_t)res & 15) == 0));
-    // Split-K into the caller's workspace.
-    const int splits = splitk_of(wide, K);
     // 256 x 128 tiles have the staged epilogue only, and no group maxima in it.
     Tile tile = tile_of(M, N, K, p.lds_epi != 0 && gmax == nullptr);
-    if (use_split(splits, K) && workspace && workspace_bytes >= splitk_bytes(M, N, K) &&
-        ((uintptr_t)workspace & 15) == 0) {
-      p.splits = splits;
+    // Split-K into the caller's workspace.
+    const size_t need = splitk_bytes(M, N, K);
+    if (need && workspace && workspace_bytes >= need && ((uintptr_t)workspace & 15) == 0) {
+      p.splits = splitk_of(M, N, K);
       p.part = static_cast<float*>(workspace);
       tile = Tile::k256x256;
     }

@@ -131,7 +131,7 @@ def _quantize_rows(x2: torch.Tensor, recipe: str):
 
 def scaled_mm(a8: torch.Tensor, sa: torch.Tensor, b8: torch.Tensor, sb: torch.Tensor) -> torch.Tensor:
     """bf16 [M, N] = (a8 [M, K] . b8 [N, K]^T) * sa[m] * sb[n] through flw_fp8_scaled_mm_ws (split
-    over K into a workspace when [M, N] has too few output tiles to fill the GPU)."""
+    over K into a workspace for a long K and an output of a third of the GPU's 256 x 256 tiles)."""
     return _lib.native().scaled_mm(a8, sa, b8, sb, None, True, _lib.stream_of(a8))
 
 

@@ -468,12 +468,6 @@ int flw_fp8_scaled_mm(const uint8_t* x8, int64_t M, int64_t K, const uint8_t* w8
                       const float* x_scale, int64_t x_scale_count, const float* w_scale,
                       int64_t w_scale_count, void* y, int64_t y_row_stride, void* stream);
 
-/* flw_fp8_scaled_mm with a workspace for a split over K, for outputs with too few 256 x 256 tiles
- * to fill the GPU (the FP8 wgrad of a linear: [N, K] outputs reduced over the tokens): each tile's
- * K range is cut into up to 8 parts whose fp32 partial sums go to the workspace and are summed,
- * scaled and rounded to bf16 by a second kernel. Same result contract as flw_fp8_scaled_mm
- * (fp32 accumulation, summed in a different order). flw_fp8_scaled_mm_workspace_bytes returns 0
- * when no split applies; with a smaller workspace the call runs unsplit. */
 /* flw_fp8_scaled_mm that also returns, for every group of group_cols consecutive output columns,
  * max |y| over all rows (as the fp32 bit pattern of the bf16 value, u32 [N / group_cols]): the
  * per-head amax of a QKV projection (group_cols = head_dim, groups ordered q heads, k heads,
@@ -506,6 +500,13 @@ int flw_fp8_scaled_mm_qk_norm_rope_amax(const uint8_t* x8, int64_t M, int64_t K,
                                         int64_t qk_cols, int qk_norm, float eps, const void* rope_cos,
                                         const void* rope_sin, int64_t seq_len, uint32_t* amax_out, void* stream);
 
+/* flw_fp8_scaled_mm with a workspace for a split over K (the FP8 wgrad of a linear: [N, K] outputs
+ * reduced over the tokens): for outputs whose 256 x 256 tiles are a third of the compute units, and
+ * K >= 12288, each tile's K range is cut into three parts whose fp32 partial sums go to the workspace
+ * and are summed, scaled and rounded to bf16 by a second kernel. Same result contract as
+ * flw_fp8_scaled_mm (fp32 accumulation, summed in a different order); without a split the result is
+ * flw_fp8_scaled_mm's bit for bit. flw_fp8_scaled_mm_workspace_bytes returns 0 when no split applies;
+ * with a smaller workspace the call runs unsplit. */
 size_t flw_fp8_scaled_mm_workspace_bytes(int64_t M, int64_t N, int64_t K);
 int flw_fp8_scaled_mm_ws(const uint8_t* x8, int64_t M, int64_t K, const uint8_t* w8, int64_t N,
                          const float* x_scale, int64_t x_scale_count, const float* w_scale,

@@ -93,6 +93,11 @@ def test_host_only_calls_work_without_a_gpu():
     assert rc == 2 and b"multiple of 64" in lib.flw_last_error()
     assert lib.flw_fp8_scaled_mm_workspace_bytes(8192, 4096, 1024) == 0    # 512 tiles: no split
     assert lib.flw_fp8_scaled_mm_workspace_bytes(256, 256, 100) == 0       # K % 128: no split
+    # a workspace only where the GEMM splits: three ranges of the fp32 output, K >= 12288 (256 compute units)
+    assert lib.flw_fp8_scaled_mm_workspace_bytes(3840, 1280, 16384) == 3 * 3840 * 1280 * 4
+    assert lib.flw_fp8_scaled_mm_workspace_bytes(3392, 1276, 12352) == 3 * 3392 * 1276 * 4
+    for shape in ((4096, 1024, 8192), (4096, 1024, 16384), (256, 256, 4096), (3840, 1280, 8192), (3840, 1280, 12296)):
+        assert lib.flw_fp8_scaled_mm_workspace_bytes(*shape) == 0, shape
     assert lib.flw_quant_cols_workspace_bytes(1000, 100) == 4 * 100 * 4   # 4 row chunks x 100 columns
     assert lib.flw_quant_cols_workspace_bytes(1000, 8) == 4 * 8 * 4
     rc = lib.flw_quant_cols_e4m3(16, 1, 100, 64, 64, _lib.SCALE_HEAD, 16, 112, 16, 16, 1 << 20, None)

@@ -57,15 +57,10 @@ def test_scaled_mm_matches_closed_form(M, N, K, sx_per_row, sw_per_col):
 @pytest.mark.parametrize("M,N,K", [(256, 256, 4096), (512, 1024, 2048), (4096, 1024, 8192), (300, 260, 1024),
                                    (100, 36, 80), (256, 256, 4160), (4096, 1024, 3392), (1024, 512, 192),
                                    (300, 260, 320), (3840, 1280, 1536), (2560, 1280, 2560)])
-def test_scaled_mm_split_k_matches_closed_form(M, N, K):
-    """flw_fp8_scaled_mm_ws: outputs with few 256 x 256 tiles are split over K into the workspace
-    (1 tile -> 8 ranges, 8 tiles -> 4, the C2 wgrad shape 64 tiles -> 4; an even split runs on
-    256 x 128 tiles with half the ranges, an odd one -- 75 tiles -> 3, 50 -> 5 -- on 256 x 256
-    tiles) and summed by the finish kernel; shapes without a split (K % 64 != 0) take the plain
-    path through the same call.
-    K % 128 == 64 (the SwiGLU width 3392 of the 450M block among them) ends the last K range on a
-    64-deep stage, in the 256 x 256 and the 256 x 128 tiles, split or not. Against the closed
-    form, and equal to the unsplit call within the GEMM tolerance."""
+def test_scaled_mm_ws_unsplit_matches_closed_form(M, N, K):
+    """flw_fp8_scaled_mm_ws where no split over K applies (no workspace is asked for, whatever one is
+    given): flw_fp8_scaled_mm's result bit for bit, and the closed form. 64 x 32 to 128 x 128 tiles, K
+    % 128 == 64 (the SwiGLU width 3392 of the 450M block among them), and K % 64 != 0."""
     from flower_amd import _lib as L
     lb = L.load()
     x8, w8 = codes((M, K), 4), codes((N, K), 5)
@@ -74,10 +69,8 @@ def test_scaled_mm_split_k_matches_closed_form(M, N, K):
     sw = rng.uniform(0.001, 0.01, N).astype(np.float32)
     tx8, tw8 = torch.from_numpy(x8).cuda(), torch.from_numpy(w8).cuda()
     tsx, tsw = torch.from_numpy(sx).cuda(), torch.from_numpy(sw).cuda()
-    need = lb.flw_fp8_scaled_mm_workspace_bytes(M, N, K)
-    if K % 64 == 0 and K >= 512 and M * N <= 8 * 256 * 256:
-        assert need > 0
-    ws = L.workspace(need, "cuda")
+    assert lb.flw_fp8_scaled_mm_workspace_bytes(M, N, K) == 0
+    ws = L.workspace(8 * M * N * 4, "cuda")
     y = torch.empty((M, N), dtype=torch.bfloat16, device="cuda")
     L.check(lb.flw_fp8_scaled_mm_ws(tx8.data_ptr(), M, K, tw8.data_ptr(), N, tsx.data_ptr(), M, tsw.data_ptr(),
                                     N, y.data_ptr(), N, ws.data_ptr(), ws.numel(), L.stream_of(y)), "mm_ws")
@@ -86,7 +79,49 @@ def test_scaled_mm_split_k_matches_closed_form(M, N, K):
     y1 = torch.empty_like(y)
     L.check(lb.flw_fp8_scaled_mm(tx8.data_ptr(), M, K, tw8.data_ptr(), N, tsx.data_ptr(), M, tsw.data_ptr(), N,
                                  y1.data_ptr(), N, L.stream_of(y)), "mm")
-    assert_gemm_close(to_np(y), to_np(y1).astype(np.float64))
+    assert torch.equal(y, y1)
+
+
+@pytest.mark.parametrize("M,N,K", [(3840, 1280, 16384), (3392, 1280, 12288), (3392, 1276, 12352), (1280, 3392, 12416)])
+@pytest.mark.parametrize("per_row", [True, False])
+def test_scaled_mm_split_k_matches_closed_form(M, N, K, per_row):
+    """flw_fp8_scaled_mm_ws where the output's 256 x 256 tiles (70 or 75) are a third of 256 compute units
+    and K >= 12288 (the 450M block's weight gradients): three K ranges' fp32 partials in the
+    workspace, of which every element is written, summed by the finish kernel. Ranges of equal and
+    unequal length, a last one that ends on a 64-deep stage, ragged rows and columns. Against the
+    closed form on sampled rows and columns, and the unsplit call; a workspace a byte short, or null,
+    runs unsplit."""
+    from flower_amd import _lib as L
+    lb = L.load()
+    if torch.cuda.get_device_properties(0).multi_processor_count != 256:
+        pytest.skip("the shapes split on 256 compute units")
+    x8, w8 = codes((M, K), 4), codes((N, K), 5)
+    rng = np.random.default_rng(6)
+    sx = rng.uniform(0.001, 0.01, M if per_row else 1).astype(np.float32)
+    sw = rng.uniform(0.001, 0.01, N if per_row else 1).astype(np.float32)
+    tx8, tw8 = torch.from_numpy(x8).cuda(), torch.from_numpy(w8).cuda()
+    tsx, tsw = torch.from_numpy(sx).cuda(), torch.from_numpy(sw).cuda()
+    need = lb.flw_fp8_scaled_mm_workspace_bytes(M, N, K)
+    assert need == 3 * M * N * 4
+
+    def call(ws, nbytes):
+        y = torch.full((M, N), 7.0, dtype=torch.bfloat16, device="cuda")
+        L.check(lb.flw_fp8_scaled_mm_ws(tx8.data_ptr(), M, K, tw8.data_ptr(), N, tsx.data_ptr(), sx.size,
+                                        tsw.data_ptr(), sw.size, y.data_ptr(), N, L.ptr(ws), nbytes,
+                                        L.stream_of(y)), "mm_ws")
+        return y
+
+    part = torch.full((3, M, N), float("nan"), device="cuda")
+    y = call(part, need)
+    assert not part.isnan().any()
+    unsplit = call(None, 0)
+    part.fill_(float("nan"))
+    assert torch.equal(call(part, need - 1), unsplit) and part.isnan().all()
+    rows = np.unique(np.r_[0, 255, 256, M - 1, rng.choice(M, 60)])
+    cols = np.unique(np.r_[0, 255, 256, N - 1, rng.choice(N, 200)])
+    ref = scaled_mm(x8[rows], w8[cols], np.broadcast_to(sx, (M,))[rows], np.broadcast_to(sw, (N,))[cols])
+    assert_gemm_close(to_np(y)[np.ix_(rows, cols)], ref)
+    assert_gemm_close(to_np(y), to_np(unsplit).astype(np.float64))
 
 
 def test_config2_fp8_linear_full_size():
