@@ -69,6 +69,26 @@ def test_ragged_columns(N, ld, K):
     assert (d <= 2.0 ** -7 * ref.abs() + 1e-3 * ref.pow(2).mean().sqrt()).all()
 
 
+# Residual rows that 16-byte loads cannot take (N or the residual's row stride 4 mod 8): the epilogue
+# without staging, on every ring tile and on the 256 x 256 tiles.
+@pytest.mark.parametrize("N,rs", [(1004, 1004), (1024, 1028)])
+@pytest.mark.parametrize("K", [320, 512])
+def test_residual_of_8_byte_rows(N, rs, K):
+    M = 13000
+    x8, w8, sx, sw = _operands(M, N, K)
+    res = torch.randn(M, rs, device="cuda").to(torch.bfloat16)[:, :N]
+    full = _rows(M, x8, w8, sx, sw, res)
+    for m in (31, 513, 1101, 2049, 4099):
+        assert torch.equal(_rows(m, x8, w8, sx, sw, res), full[:m]), m
+    for r in (slice(0, 64), slice(M - 64, M)):
+        prod = (x8.view(torch.float8_e4m3fn)[r].double() * sx[r, None]) @ (
+            w8.view(torch.float8_e4m3fn).double() * sw[:, None]).t().contiguous()
+        ref = prod + res[r].double()
+        # the product's and the sum's bf16 rounding, half a step each, and fp32 sums of 512 products
+        bound = 2.0 ** -8 * (ref.abs() + 2 * prod.abs()) + 1e-3 * prod.pow(2).mean().sqrt()
+        assert ((full[r].double() - ref).abs() <= bound).all()
+
+
 @pytest.mark.parametrize("gcols", [8, 64, 128])
 def test_group_maxima_of_every_tile(gcols):
     x8, w8, sx, sw = _operands(13000, 1152, 256)
