@@ -588,14 +588,13 @@ __device__ __forceinline__ void gemm_tile(const GemmParams& p, uint8_t* st0, uin
   }
 }
 
-// One 256 (n) x 128 (m) output tile (or its K range under split-K), for outputs with fewer
-// 256 x 256 tiles than compute units (twice the tiles, so the grid covers more of the GPU): 8 waves in a 4 x 2 grid of 64 x 64 wave tiles
-// (2 x 2 MFMAs per 64-deep K chunk), a stage holding the 256 W rows and 128 X rows (48 of its
+// One 256 (n) x 128 (m) output tile, for outputs whose rounds of 256 x 256 tiles fill the GPU worse
+// (tile_of): 8 waves in a 4 x 2 grid of 64 x 64 wave tiles (2 x 2 MFMAs per 64-deep K chunk), a stage holding the 256 W rows and 128 X rows (48 of its
 // 64 KB), the same swizzle, barriers and accumulation order as gemm_tile (the results are
 // identical), and the epilogue staged through st0 (128 rows x 512 bytes).
 template <bool HALFK = false>
 __device__ __forceinline__ void gemm_tile_128(const GemmParams& p, uint8_t* st0, uint8_t* st1, int m0,
-                                              int n0, int wave, int lane, int sbase, int nst, int split) {
+                                              int n0, int wave, int lane, int nst) {
   const int wn = wave & 3, wm = wave >> 2;        // 64 n rows, 64 m columns
   // Loads: 384 rows of 128 bytes per stage; wave w fills rows 48 w .. 48 w + 47 with 6
   // instructions of 8 rows, rows 256 .. 383 being X rows 0 .. 127. Instruction t of a wave reads
@@ -612,10 +611,9 @@ __device__ __forceinline__ void gemm_tile_128(const GemmParams& p, uint8_t* st0,
     goff[t] = (uint32_t)grow * (uint32_t)p.K + 16u * (uint32_t)c;
     hi_half |= (uint32_t)(c >> 2) << t;
   }
-  const bool half_last = HALFK && sbase + nst == (p.K + kFBK - 1) / kFBK;
   auto issue = [&](uint8_t* stage, int s) __attribute__((always_inline)) {
-    const uint32_t k0 = (uint32_t)(sbase + s) * kFBK;
-    const uint32_t back = half_last && s == nst - 1 ? 64u : 0u;
+    const uint32_t k0 = (uint32_t)s * kFBK;
+    const uint32_t back = HALFK && s == nst - 1 ? 64u : 0u;
     const uint32_t lds = (uint32_t)(uintptr_t)(lds_u8_t*)stage;
 #pragma unroll
     for (int t = 0; t < 6; ++t) {
@@ -646,7 +644,7 @@ __device__ __forceinline__ void gemm_tile_128(const GemmParams& p, uint8_t* st0,
     lds_barrier();                                // ... and every wave's
 #pragma unroll
     for (int kc = 0; kc < 2; ++kc) {
-      if (kc == 1 && half_last && s == nst - 1) break;      // a 64-deep last stage
+      if (HALFK && kc == 1 && s == nst - 1) break;      // a 64-deep last stage
       v8i a[2], b[2];
 #pragma unroll
       for (int i = 0; i < 2; ++i) a[i] = swz_frag(cur, 2 * wn + i, kc, lane);
@@ -667,28 +665,8 @@ __device__ __forceinline__ void gemm_tile_128(const GemmParams& p, uint8_t* st0,
 
   // Epilogue: lane owns m = m0 + 64 wm + 32 j + lane % 32, n = n0 + 64 wn + 32 i + 8 g + 4 hh + 0..3;
   // the scaled bf16 tile goes to st0 (row r = m - m0, 16-byte chunk c at c ^ (r & 31)), then
-  // wave w stores rows 16 w .. 16 w + 15, two 512-byte rows per instruction. Split-K: unscaled
-  // fp32 partials, 16-byte stores.
+  // wave w stores rows 16 w .. 16 w + 15, two 512-byte rows per instruction.
   const int hh = lane >> 5;
-  if (p.part) {
-    float* base = p.part + (int64_t)split * p.M * p.N;
-#pragma unroll
-    for (int i = 0; i < 2; ++i)
-#pragma unroll
-      for (int j = 0; j < 2; ++j) {
-        const int m = m0 + 64 * wm + 32 * j + (lane & 31);
-        if (m >= p.M) continue;
-#pragma unroll
-        for (int g = 0; g < 4; ++g) {
-          const int n = n0 + 64 * wn + 32 * i + 8 * g + 4 * hh;
-          if (n >= p.N) continue;
-          const v16f& c = acc[i][j];
-          *reinterpret_cast<float4*>(base + (int64_t)m * p.N + n) =
-              make_float4(c[4 * g], c[4 * g + 1], c[4 * g + 2], c[4 * g + 3]);
-        }
-      }
-    return;
-  }
   float sxm[2];
 #pragma unroll
   for (int j = 0; j < 2; ++j) {
@@ -781,7 +759,7 @@ __global__ __launch_bounds__(kFThreads, 1) void fp8_gemm_256_kernel(GemmParams p
     const int tn = (tt % (kGroupM * p.tiles_n)) / gm;
     const int s0 = split * nst_all / p.splits, s1 = (split + 1) * nst_all / p.splits;
     if constexpr (TM == 256) gemm_tile<XD, HALFK>(p, st0, st1, tm * kFBM, tn * kFBN, wave, lane, s0, s1 - s0, split);
-    else gemm_tile_128<HALFK>(p, st0, st1, tm * TM, tn * kFBN, wave, lane, s0, s1 - s0, split);
+    else gemm_tile_128<HALFK>(p, st0, st1, tm * TM, tn * kFBN, wave, lane, nst_all);   // never split
   }
 }
 
@@ -810,29 +788,11 @@ __device__ __forceinline__ void unrolled_down(F f) {
 // n = 32 (TN wn + i) + 8 g + 4 (lane / 32) + 0..3.
 template <int WN, int WM, int TN, int TM, int XD>
 __device__ __forceinline__ void ring_epilogue(const GemmParams& p, const v16f (&acc)[TN][TM], uint8_t* lds, int m0,
-                                              int n0, int wave, int lane, int split) {
+                                              int n0, int wave, int lane) {
   constexpr int BN = 32 * WN * TN, BM = 32 * WM * TM, NW = WN * WM;
   constexpr int CPR = BN / 8;                     // 16-byte chunks of a row
   constexpr int ROWB = BN * 2;
   const int wn = wave % WN, wm = wave / WN, hh = lane >> 5, tid = wave * 64 + lane;
-  if (p.part) {                                   // split-K: unscaled fp32 partials, 16-byte stores
-    float* base = p.part + (int64_t)split * p.M * p.N;
-#pragma unroll
-    for (int i = 0; i < TN; ++i)
-#pragma unroll
-      for (int j = 0; j < TM; ++j) {
-        const int m = m0 + 32 * (TM * wm + j) + (lane & 31);
-#pragma unroll
-        for (int g = 0; g < 4; ++g) {
-          const int n = n0 + 32 * (TN * wn + i) + 8 * g + 4 * hh;
-          const v16f& c = acc[i][j];
-          if (m < p.M && n < p.N)
-            *reinterpret_cast<float4*>(base + (int64_t)m * p.N + n) =
-                make_float4(c[4 * g], c[4 * g + 1], c[4 * g + 2], c[4 * g + 3]);
-        }
-      }
-    return;
-  }
 #pragma unroll
   for (int i = 0; i < TN; ++i) {
     float swn[16];
@@ -1002,9 +962,6 @@ __device__ __forceinline__ void ring_epilogue(const GemmParams& p, const v16f (&
       atomicMax(p.gmax + (n0 + 8 * lpg * tid) / p.gcols, mx << 16);     // bf16 bits -> fp32 bits
     }
   }
-  // The next tile's loads refill the ring: every wave's reads of the staged tile are done.
-  __builtin_amdgcn_s_waitcnt(0xC07F);
-  lds_barrier();
 }
 
 template <int WN, int WM, int TN, int TM, int NST, int XD = 0, bool HALFK = false, bool PIPE = false>
@@ -1020,136 +977,130 @@ __global__ __launch_bounds__(64 * WN * WM) void fp8_gemm_ring_kernel(GemmParams 
   const int wn = wave % WN, wm = wave / WN;
   const uint32_t lds0 = (uint32_t)(uintptr_t)(lds_u8_t*)lds;
   const uint8_t *const w8 = p.w8, *const x8 = p.x8;
-  const int nst_all = (p.K + kFBK - 1) / kFBK;    // the last one 64 deep when K % 128 == 64
+  const int nst = (p.K + kFBK - 1) / kFBK;        // the last one 64 deep when K % 128 == 64
+  // One tile a workgroup; consecutive tiles on one XCD.
   const int G = gridDim.x;
-  const int L = (G & 7) == 0 ? (blockIdx.x & 7) * (G >> 3) + (blockIdx.x >> 3) : blockIdx.x;
-  const int ntiles = p.tiles_n * p.tiles_m;
-  for (int item = L; item < ntiles * p.splits; item += G) {
-    const int split = item / ntiles, t = item % ntiles;
-    const int group = t / (kGroupM * p.tiles_n);
-    const int first_m = group * kGroupM;
-    const int gm = min(p.tiles_m - first_m, kGroupM);
-    const int m0 = (first_m + (t % (kGroupM * p.tiles_n)) % gm) * BM;
-    const int n0 = ((t % (kGroupM * p.tiles_n)) / gm) * BN;
-    // Split-K: this item's K stages.
-    const int sbase = split * nst_all / p.splits, nst = (split + 1) * nst_all / p.splits - sbase;
-    const bool half_last = HALFK && sbase + nst == nst_all;
-    // Lane i of instruction q fetches row 8 q + i / 8 of the wave's rows, LDS position i % 8, i.e.
-    // global chunk (i % 8) ^ swizzle; rows past M / N fetch the last valid row (not stored).
-    uint32_t goff[IPW];
-    uint32_t hi_half = 0;                         // bit q: instruction q's chunk is in bytes 64-127
+  const int t = (G & 7) == 0 ? (blockIdx.x & 7) * (G >> 3) + (blockIdx.x >> 3) : blockIdx.x;
+  const int group = t / (kGroupM * p.tiles_n);
+  const int first_m = group * kGroupM;
+  const int gm = min(p.tiles_m - first_m, kGroupM);
+  const int m0 = (first_m + (t % (kGroupM * p.tiles_n)) % gm) * BM;
+  const int n0 = ((t % (kGroupM * p.tiles_n)) / gm) * BN;
+  // Lane i of instruction q fetches row 8 q + i / 8 of the wave's rows, LDS position i % 8, i.e.
+  // global chunk (i % 8) ^ swizzle; rows past M / N fetch the last valid row (not stored).
+  uint32_t goff[IPW];
+  uint32_t hi_half = 0;                         // bit q: instruction q's chunk is in bytes 64-127
+#pragma unroll
+  for (int q = 0; q < IPW; ++q) {
+    const int row0 = 8 * (wave * IPW + q);
+    const bool xop = row0 >= BN;
+    const int r = (xop ? row0 - BN : row0) + (lane >> 3);
+    const int c = (lane & 7) ^ ((r >> 1) & 7);
+    const int grow = xop ? min(m0 + r, p.M - 1) : min(n0 + r, p.N - 1);
+    goff[q] = (uint32_t)grow * (uint32_t)p.K + 16u * (uint32_t)c;
+    hi_half |= (uint32_t)(c >> 2) << q;
+  }
+  auto issue = [&](int s) __attribute__((always_inline)) {
+    const uint32_t dst = lds0 + (uint32_t)(s % NST) * kStage;
+    const uint32_t back = HALFK && s == nst - 1 ? 64u : 0u;   // the last stage's bytes 64-127: 0-63 again
 #pragma unroll
     for (int q = 0; q < IPW; ++q) {
       const int row0 = 8 * (wave * IPW + q);
-      const bool xop = row0 >= BN;
-      const int r = (xop ? row0 - BN : row0) + (lane >> 3);
-      const int c = (lane & 7) ^ ((r >> 1) & 7);
-      const int grow = xop ? min(m0 + r, p.M - 1) : min(n0 + r, p.N - 1);
-      goff[q] = (uint32_t)grow * (uint32_t)p.K + 16u * (uint32_t)c;
-      hi_half |= (uint32_t)(c >> 2) << q;
+      const uint8_t* src = row0 >= BN ? x8 : w8;
+      asm volatile("s_mov_b32 m0, %0\n\tglobal_load_lds_dwordx4 %1, %2"
+                   :: "s"(dst + row0 * 128), "v"(goff[q] + (uint32_t)s * kFBK - (((hi_half >> q) & 1u) ? back : 0u)),
+                      "s"(src) : "memory", "m0");
     }
-    auto issue = [&](int s) __attribute__((always_inline)) {
-      const uint32_t dst = lds0 + (uint32_t)(s % NST) * kStage;
-      const uint32_t back = half_last && s == nst - 1 ? 64u : 0u;   // the last stage's bytes 64-127: 0-63 again
+  };
+  v16f acc[TN][TM];
 #pragma unroll
-      for (int q = 0; q < IPW; ++q) {
-        const int row0 = 8 * (wave * IPW + q);
-        const uint8_t* src = row0 >= BN ? x8 : w8;
-        asm volatile("s_mov_b32 m0, %0\n\tglobal_load_lds_dwordx4 %1, %2"
-                     :: "s"(dst + row0 * 128), "v"(goff[q] + (uint32_t)(sbase + s) * kFBK - (((hi_half >> q) & 1u) ? back : 0u)),
-                        "s"(src) : "memory", "m0");
-      }
-    };
-    v16f acc[TN][TM];
+  for (int i = 0; i < TN; ++i)
+#pragma unroll
+    for (int j = 0; j < TM; ++j) acc[i][j] = v16f{};
+#pragma unroll
+  for (int s = 0; s < NST - 1; ++s)
+    if (s < nst) issue(s);
+  v8i a[2][2][TN], b[2][2][TM];                 // fragments [parity][K chunk][block]
+  auto read = [&](int s, auto pc) __attribute__((always_inline)) {
+    constexpr int P = decltype(pc)::value;
+    const uint8_t* cur = lds + (s % NST) * kStage;
+#pragma unroll
+    for (int kc = 0; kc < 2; ++kc) {
+#pragma unroll
+      for (int i = 0; i < TN; ++i) a[P][kc][i] = swz_frag(cur, TN * wn + i, kc, lane);
+#pragma unroll
+      for (int j = 0; j < TM; ++j) b[P][kc][j] = swz_frag(cur, BN / 32 + TM * wm + j, kc, lane);
+    }
+  };
+  auto prod = [&](auto pc, auto kcc) __attribute__((always_inline)) {
+    constexpr int P = decltype(pc)::value, kc = decltype(kcc)::value;
 #pragma unroll
     for (int i = 0; i < TN; ++i)
 #pragma unroll
-      for (int j = 0; j < TM; ++j) acc[i][j] = v16f{};
-#pragma unroll
-    for (int s = 0; s < NST - 1; ++s)
-      if (s < nst) issue(s);
-    v8i a[2][2][TN], b[2][2][TM];                 // fragments [parity][K chunk][block]
-    auto read = [&](int s, auto pc) __attribute__((always_inline)) {
-      constexpr int P = decltype(pc)::value;
-      const uint8_t* cur = lds + (s % NST) * kStage;
-#pragma unroll
-      for (int kc = 0; kc < 2; ++kc) {
-#pragma unroll
-        for (int i = 0; i < TN; ++i) a[P][kc][i] = swz_frag(cur, TN * wn + i, kc, lane);
-#pragma unroll
-        for (int j = 0; j < TM; ++j) b[P][kc][j] = swz_frag(cur, BN / 32 + TM * wm + j, kc, lane);
+      for (int j = 0; j < TM; ++j) acc[i][j] = gemm_mfma(a[P][kc][i], b[P][kc][j], acc[i][j]);
+  };
+  using C0 = std::integral_constant<int, 0>;
+  using C1 = std::integral_constant<int, 1>;
+  auto mult = [&](int s, bool last) __attribute__((always_inline)) {
+    read(s, C0{});
+    prod(C0{}, C0{});
+    if (!(HALFK && last)) prod(C0{}, C1{});
+    __builtin_amdgcn_s_waitcnt(0xC07F);         // lgkmcnt(0): this wave's reads of stage s are done
+  };
+  auto fetch = [&](int s, auto pc) __attribute__((always_inline)) {
+    __builtin_amdgcn_s_waitcnt(vmcnt_imm((NST - 2) * IPW));   // this wave's loads of stage s landed
+    lds_barrier();                              // ... and every wave's; stage s - 1 is retired
+    issue(s + NST - 1);
+    read(s, pc);
+  };
+  if constexpr (PIPE) {
+    if (nst >= NST) {
+      int s = 0;
+      fetch(0, C0{});
+#pragma unroll 1
+      for (; s + NST + 1 < nst; s += 2) {
+        __builtin_amdgcn_s_waitcnt(0xC07F);
+        prod(C0{}, C0{});
+        fetch(s + 1, C1{});
+        prod(C0{}, C1{});
+        __builtin_amdgcn_s_waitcnt(0xC07F);
+        prod(C1{}, C0{});
+        fetch(s + 2, C0{});
+        prod(C1{}, C1{});
       }
-    };
-    auto prod = [&](auto pc, auto kcc) __attribute__((always_inline)) {
-      constexpr int P = decltype(pc)::value, kc = decltype(kcc)::value;
-#pragma unroll
-      for (int i = 0; i < TN; ++i)
-#pragma unroll
-        for (int j = 0; j < TM; ++j) acc[i][j] = gemm_mfma(a[P][kc][i], b[P][kc][j], acc[i][j]);
-    };
-    using C0 = std::integral_constant<int, 0>;
-    using C1 = std::integral_constant<int, 1>;
-    auto mult = [&](int s, bool last) __attribute__((always_inline)) {
-      read(s, C0{});
+      __builtin_amdgcn_s_waitcnt(0xC07F);
       prod(C0{}, C0{});
-      if (!(half_last && last)) prod(C0{}, C1{});
-      __builtin_amdgcn_s_waitcnt(0xC07F);         // lgkmcnt(0): this wave's reads of stage s are done
-    };
-    auto fetch = [&](int s, auto pc) __attribute__((always_inline)) {
+      if (s + NST < nst) {
+        fetch(s + 1, C1{});
+        prod(C0{}, C1{});
+        __builtin_amdgcn_s_waitcnt(0xC07F);
+        prod(C1{}, C0{});
+        prod(C1{}, C1{});
+      } else {
+        prod(C0{}, C1{});
+      }
+    }
+  } else {
+#pragma unroll 1
+    for (int s = 0; s + NST - 1 < nst; ++s) {
       __builtin_amdgcn_s_waitcnt(vmcnt_imm((NST - 2) * IPW));   // this wave's loads of stage s landed
       lds_barrier();                              // ... and every wave's; stage s - 1 is retired
       issue(s + NST - 1);
-      read(s, pc);
-    };
-    if constexpr (PIPE) {
-      if (nst >= NST) {
-        int s = 0;
-        fetch(0, C0{});
-#pragma unroll 1
-        for (; s + NST + 1 < nst; s += 2) {
-          __builtin_amdgcn_s_waitcnt(0xC07F);
-          prod(C0{}, C0{});
-          fetch(s + 1, C1{});
-          prod(C0{}, C1{});
-          __builtin_amdgcn_s_waitcnt(0xC07F);
-          prod(C1{}, C0{});
-          fetch(s + 2, C0{});
-          prod(C1{}, C1{});
-        }
-        __builtin_amdgcn_s_waitcnt(0xC07F);
-        prod(C0{}, C0{});
-        if (s + NST < nst) {
-          fetch(s + 1, C1{});
-          prod(C0{}, C1{});
-          __builtin_amdgcn_s_waitcnt(0xC07F);
-          prod(C1{}, C0{});
-          prod(C1{}, C1{});
-        } else {
-          prod(C0{}, C1{});
-        }
-      }
-    } else {
-#pragma unroll 1
-      for (int s = 0; s + NST - 1 < nst; ++s) {
-        __builtin_amdgcn_s_waitcnt(vmcnt_imm((NST - 2) * IPW));   // this wave's loads of stage s landed
-        lds_barrier();                              // ... and every wave's; stage s - 1 is retired
-        issue(s + NST - 1);
-        mult(s, false);
-      }
+      mult(s, false);
     }
-    // The last NST - 1 stages: nothing left to issue, r stages still in flight behind each.
-    auto tail = [&](auto rc) __attribute__((always_inline)) {
-      constexpr int r = decltype(rc)::value;
-      if (r < nst) {
-        __builtin_amdgcn_s_waitcnt(vmcnt_imm(r * IPW));
-        lds_barrier();
-        mult(nst - 1 - r, r == 0);
-      }
-    };
-    unrolled_down<NST - 2>(tail);
-    lds_barrier();                                // the epilogue overwrites the ring
-    ring_epilogue<WN, WM, TN, TM, XD>(p, acc, lds, m0, n0, wave, lane, split);
   }
+  // The last NST - 1 stages: nothing left to issue, r stages still in flight behind each.
+  auto tail = [&](auto rc) __attribute__((always_inline)) {
+    constexpr int r = decltype(rc)::value;
+    if (r < nst) {
+      __builtin_amdgcn_s_waitcnt(vmcnt_imm(r * IPW));
+      lds_barrier();
+      mult(nst - 1 - r, r == 0);
+    }
+  };
+  unrolled_down<NST - 2>(tail);
+  lds_barrier();                                // the epilogue overwrites the ring
+  ring_epilogue<WN, WM, TN, TM, XD>(p, acc, lds, m0, n0, wave, lane);
 }
 
 // Split-K finish: y[m, n..n+3] = bf16( (sum_s part[s][m][n]) * sx[m] * sw[n] ) (+ residual as in
@@ -1486,7 +1437,10 @@ __global__ __launch_bounds__(64 * WN * WM) void w8a16_ring_kernel(W8A16Params p)
     };
     unrolled_down<NST - 2>(tail);
     lds_barrier();                                // the epilogue overwrites the ring
-    ring_epilogue<WN, WM, TN, TM, 0>(e, acc, lds, m0, n0, wave, lane, 0);
+    ring_epilogue<WN, WM, TN, TM, 0>(e, acc, lds, m0, n0, wave, lane);
+    // The next tile's loads refill the ring: every wave's reads of the staged tile are done.
+    __builtin_amdgcn_s_waitcnt(0xC07F);
+    lds_barrier();
   }
 }
 
@@ -1523,7 +1477,7 @@ static size_t splitk_bytes(int64_t M, int64_t N, int64_t K) {
 enum class Tile { k64x32, k64x64, k128x64, k128x128, k128x128Pair, k256x128, k256x256 };
 
 // The tile for an [M, N] output (K % 64 == 0). While one of the smaller tiles gives at most one tile
-// per compute unit, the largest such: a tile's time hardly depends on how many others run (K =
+// per compute unit, the smallest such: a tile's time hardly depends on how many others run (K =
 // 4096, us: 8.5 / 9 / 10.5 / 15 / 28 / 48 for 64x32 / 64x64 / 128x64 / 128x128 / 256x128 / 256x256),
 // so a small output takes the smallest that fits in one round ([16, 1024] at K = 4096 28 -> 8.2 us,
 // [2048, 1024] 30 -> 13.4 us, [1024, 3072] at K = 1024 11.0 -> 8.0 us). Up to two 128 x 128 tiles
@@ -1548,7 +1502,8 @@ static Tile tile_of(int64_t M, int64_t N, int64_t K, bool narrow_ok) {
 
 struct TileKernel {
   const void* fn;
-  int bn, bm, threads, per_cu;        // per_cu: workgroups that fit a compute unit's LDS
+  int bn, bm, threads;
+  int per_cu;                         // workgroups a compute unit holds of a persistent kernel; 0: one a tile
 };
 
 // XD: head dim of the q / k transform epilogue (0: none; HALFK never set with it).
@@ -1557,21 +1512,21 @@ static TileKernel tile_kernel(Tile t) {
   switch (t) {
     case Tile::k64x32:
       if constexpr (XD == 0)
-        return {reinterpret_cast<const void*>(&fp8_gemm_ring_kernel<2, 1, 1, 1, 4, 0, HALFK>), 64, 32, 128, 3};
+        return {reinterpret_cast<const void*>(&fp8_gemm_ring_kernel<2, 1, 1, 1, 4, 0, HALFK>), 64, 32, 128, 0};
       [[fallthrough]];
     case Tile::k64x64:
       if constexpr (XD == 0)
-        return {reinterpret_cast<const void*>(&fp8_gemm_ring_kernel<2, 2, 1, 1, 4, 0, HALFK, true>), 64, 64, 256, 2};
+        return {reinterpret_cast<const void*>(&fp8_gemm_ring_kernel<2, 2, 1, 1, 4, 0, HALFK, true>), 64, 64, 256, 0};
       [[fallthrough]];
     case Tile::k128x64:
       if constexpr (XD == 0)
-        return {reinterpret_cast<const void*>(&fp8_gemm_ring_kernel<4, 2, 1, 1, 4, 0, HALFK, true>), 128, 64, 512, 1};
+        return {reinterpret_cast<const void*>(&fp8_gemm_ring_kernel<4, 2, 1, 1, 4, 0, HALFK, true>), 128, 64, 512, 0};
       else    // 16 rows a wave, whole row batches of the head-major epilogue
-        return {reinterpret_cast<const void*>(&fp8_gemm_ring_kernel<2, 2, 2, 1, 3, XD, HALFK, true>), 128, 64, 256, 2};
+        return {reinterpret_cast<const void*>(&fp8_gemm_ring_kernel<2, 2, 2, 1, 3, XD, HALFK, true>), 128, 64, 256, 0};
     case Tile::k128x128:
-      return {reinterpret_cast<const void*>(&fp8_gemm_ring_kernel<4, 2, 1, 2, 3, XD, HALFK, true>), 128, 128, 512, 1};
+      return {reinterpret_cast<const void*>(&fp8_gemm_ring_kernel<4, 2, 1, 2, 3, XD, HALFK, true>), 128, 128, 512, 0};
     case Tile::k128x128Pair:
-      return {reinterpret_cast<const void*>(&fp8_gemm_ring_kernel<4, 2, 1, 2, 2, XD, HALFK>), 128, 128, 512, 2};
+      return {reinterpret_cast<const void*>(&fp8_gemm_ring_kernel<4, 2, 1, 2, 2, XD, HALFK>), 128, 128, 512, 0};
     case Tile::k256x128:
       if constexpr (XD == 0)
         return {reinterpret_cast<const void*>(&fp8_gemm_256_kernel<128, 0, HALFK>), 256, 128, kFThreads, 1};
@@ -1627,9 +1582,9 @@ static int scaled_mm(const uint8_t* x8, int64_t M, int64_t K, const uint8_t* w8,
     const int64_t tiles_n = (N + k.bn - 1) / k.bn, tiles_m = (M + k.bm - 1) / k.bm;
     p.tiles_n = (int)tiles_n;
     p.tiles_m = (int)tiles_m;
-    // Persistent: as many workgroups as the compute units hold at once, at most one per work item.
-    const int64_t items = tiles_n * tiles_m * p.splits, slots = (int64_t)compute_units() * k.per_cu;
-    FLW_REQUIRE(items <= 0x7FFFFFFF - slots, FLW_E_UNSUPPORTED, "grid too large");
+    // Persistent kernels: as many workgroups as the compute units hold at once, at most one per work item.
+    const int64_t items = tiles_n * tiles_m * p.splits, slots = k.per_cu ? (int64_t)compute_units() * k.per_cu : items;
+    FLW_REQUIRE(items <= 0x7FFFFFFF - compute_units(), FLW_E_UNSUPPORTED, "grid too large");
     const dim3 grid((unsigned)(items < slots ? items : slots)), block((unsigned)k.threads);
     if (gmax) {
       FLW_REQUIRE(p.splits == 1 && p.lds_epi, FLW_E_UNSUPPORTED,
