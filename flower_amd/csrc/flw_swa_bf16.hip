@@ -61,12 +61,12 @@ struct SwaB16Params {
   float* delta;           // [B, H, T]
   int H, T, W, nblk, nwg; // nblk: 128-row blocks per (b, h)
   int ramp;               // query blocks per slice whose band is cut short by the sequence's start
-  int ramp_k;             // key blocks per slice whose band is cut short by its end
   int group_slices;       // slices per dispatch group (one XCD's share when it is whole slices)
-  int wg0;                // backward kernel: the launch's first workgroup, of 2 nwg
   float sm_scale;
   int64_t rows;           // B * H * T (delta kernel)
   int o_tmaj;             // O and dO token-major, (B, T, H, D): rows of a (b, h) slice H D apart
+  int ramp_k;             // backward: key blocks per slice whose band is cut short by the sequence's end
+  int wg0;                // backward kernel: the launch's first workgroup, of 2 nwg
 };
 
 // O / dO of slice (b, h) = bh: its first row and its row stride in elements. Head-major (B, H, T, D)
