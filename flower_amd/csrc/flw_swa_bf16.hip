@@ -678,11 +678,12 @@ __device__ __forceinline__ void dq_block(const SwaB16Params& p, int wg, TilePair
 // large ones while the last blocks drain. Backward (Delta included), two launches -> one, us:
 // D = 64: B1 H8 T1500 W500 33.6 -> 23.4, B1 H20 T4096 W2048 143 -> 131, B2 H20 T8192 W2048 552 -> 520;
 // D = 32: B1 H8 T1500 W500 26.0 -> 16.7; D = 128: B1 H8 T1500 W500 50.4 -> 31.8. The same bits.
-// The tiles' LDS: one array at D = 32 and 64, which the register allocator takes 166 VGPRs for at
-// D = 64, three waves a SIMD (as two arrays 176, two waves: 553 us at T8192), two at D = 128, where
-// one wave runs either way (one array: 33 us at T1500, 1251 against 1215 at B2 H20 T8192 W2048).
+// Waves a SIMD: four at D = 32 (118 VGPRs), three at D = 64 (164), as the launch bounds ask, one at D =
+// 128. At D = 64 a bound of two left it to the allocator, which gave three waves with the tiles' LDS
+// as one array and two (176 VGPRs, 553 us at T8192) as two arrays. At D = 128, where one wave runs
+// either way, two arrays (one: 33 us at T1500, 1251 against 1215 at B2 H20 T8192 W2048).
 template <int D>
-__global__ __launch_bounds__(256, D == 128 ? 1 : 2) void swa_bf16_bwd_kernel(SwaB16Params p) {
+__global__ __launch_bounds__(256, D == 128 ? 1 : D == 64 ? 3 : 4) void swa_bf16_bwd_kernel(SwaB16Params p) {
   __shared__ __align__(16) TilePair<D> t[D == 128 ? 1 : 2];
   __shared__ __align__(16) float stat[2][2][64];
   auto run = [&](TilePair<D>& a, TilePair<D>& b) __attribute__((always_inline)) {
