@@ -81,7 +81,8 @@ def _native_cmd(out: str) -> list:
     libdir = os.path.join(os.path.dirname(torch.__file__), "lib")
     inc = [*cpp_extension.include_paths(), sysconfig.get_paths()["include"]]
     return [shutil.which("g++") or "g++", "-O2", "-std=c++17", "-fPIC", "-shared", "-fvisibility=hidden",
-            f"-D_GLIBCXX_USE_CXX11_ABI={int(torch._C._GLIBCXX_USE_CXX11_ABI)}", *(f"-I{d}" for d in inc), NATIVE_SOURCE,
+            f"-D_GLIBCXX_USE_CXX11_ABI={int(torch._C._GLIBCXX_USE_CXX11_ABI)}",
+            f'-DFLW_TORCH_VERSION="{torch.__version__}"', *(f"-I{d}" for d in inc), NATIVE_SOURCE,
             "-o", out, "-L", HERE, "-l:libflower_amd.so", "-L", libdir, "-lc10", "-ltorch_cpu", "-ltorch_python",
             "-Wl,-rpath,$ORIGIN"]
 

@@ -238,13 +238,21 @@ _native_mod = None
 
 def native():
     """flower_amd._native: the operators' allocate-and-launch bodies in C++ (csrc/native/flw_host.cpp),
-    over the same C ABI; they raise ValueError / FlowerError as ``check`` does."""
+    over the same C ABI; they raise ValueError / FlowerError as ``check`` does. The extension is tied to
+    the torch and Python it was built with; any other is refused here."""
     global _native_mod
     if _native_mod is None:
         load()
         if not os.path.exists(NATIVE_PATH):
             raise RuntimeError(f"_native.so is not built ({NATIVE_PATH}); run `python -m flower_amd._build`")
-        from . import _native
+        try:
+            from . import _native
+            built = getattr(_native, "torch_version", "another torch")
+        except ImportError as e:
+            built = e
+        if built != str(torch.__version__):
+            raise RuntimeError(f"_native.so was not built with this Python and torch {torch.__version__} ({built}); "
+                               "run `python -m flower_amd._build`")
         _native_mod = _native
     return _native_mod
 

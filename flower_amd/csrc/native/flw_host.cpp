@@ -390,6 +390,7 @@ std::tuple<Tensor, Tensor> qkv_norm_rope_amax(const Tensor& a8, const Tensor& sa
 }  // namespace
 
 PYBIND11_MODULE(_native, m) {
+  m.attr("torch_version") = FLW_TORCH_VERSION;   // compared at load: tensors cross here in that build's layout
   py::register_exception_translator([](std::exception_ptr p) {
     try {
       if (p) std::rethrow_exception(p);

@@ -345,3 +345,17 @@ def test_training_row_kernel_refusals_on_the_host():
     assert rc == 3 and b"workspace" in lib.flw_last_error()
     rc = lib.flw_quant_tensor_t_e4m3(P, 0, 1280, 1280, P, 1280, P, 1024, P, P, need, None)
     assert rc == 1 and b"empty" in lib.flw_last_error()
+
+
+def test_native_extension_of_another_torch_is_refused(monkeypatch):
+    """The extension's functions take tensors in the layout of the torch it was built with."""
+    import torch
+
+    from flower_amd import _lib
+    if not os.path.exists(_lib.NATIVE_PATH):
+        pytest.skip("_native.so not built (run __graft_entry__.build())")
+    _lib.native()
+    monkeypatch.setattr(_lib, "_native_mod", None)
+    monkeypatch.setattr(torch, "__version__", "0.0.0")
+    with pytest.raises(RuntimeError, match="not built with this Python and torch 0.0.0"):
+        _lib.native()
