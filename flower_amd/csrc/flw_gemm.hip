@@ -589,9 +589,10 @@ __device__ __forceinline__ void gemm_tile(const GemmParams& p, uint8_t* st0, uin
 }
 
 // One 256 (n) x 128 (m) output tile, for outputs whose rounds of 256 x 256 tiles fill the GPU worse
-// (tile_of): 8 waves in a 4 x 2 grid of 64 x 64 wave tiles (2 x 2 MFMAs per 64-deep K chunk), a stage holding the 256 W rows and 128 X rows (48 of its
-// 64 KB), the same swizzle, barriers and accumulation order as gemm_tile (the results are
-// identical), and the epilogue staged through st0 (128 rows x 512 bytes).
+// (tile_of): 8 waves in a 4 x 2 grid of 64 x 64 wave tiles (2 x 2 MFMAs per 64-deep K chunk), a stage
+// holding the 256 W rows and 128 X rows (48 of its 64 KB), the same swizzle, barriers and accumulation
+// order as gemm_tile (the results are identical), and the epilogue staged through st0 (128 rows x 512
+// bytes).
 template <bool HALFK = false>
 __device__ __forceinline__ void gemm_tile_128(const GemmParams& p, uint8_t* st0, uint8_t* st1, int m0,
                                               int n0, int wave, int lane, int nst) {
@@ -1458,10 +1459,12 @@ static bool tiled(int64_t M, int64_t N, int64_t K) {
 }
 
 // K ranges per 256 x 256 output tile, for the workspace query and the GEMM alike: three where that many
-// fill the GPU and K is long enough to pay for the partials ([3840, 1280] and [3392, 1280] at K = 16384
-// 93 / 90 us against 102 / 99 us unsplit, 61 / 59 against 53 / 52 us at K = 8192), one otherwise. Two
-// ranges, or four and more, measured slower than the smaller tiles unsplit: [4096, 1024] at K = 8192 48
-// -> 37 us, [1024, 1024] at K = 4096 24 -> 10 us.
+// fill the GPU and K is long enough to pay for the partials, one otherwise. Unsplit against split, us:
+// three ranges, K = 8192 / 10240 / 12288 / 16384: [3392, 1280] 56 / 71 / 82 / 103 against 62 / 73 / 80
+// / 96, [3840, 1280] 57 / 72 / 86 / 103 against 64 / 75 / 83 / 100, [4096, 1280] 58 / 73 / 100 / 113
+// against 66 / 75 / 85 / 102, [4352, 1024] 58 / 73 / 85 / 109 against 62 / 73 / 80 / 98. Four at K =
+// 8192 / 16384: [4096, 1024] 39 / 75 against 50 / 84, [3072, 1280] 37 / 73 against 48 / 81; two: [5120,
+// 1280] 62 / 121 against 64 / 123; eight: [1024, 1024] 17 / 30 against 28 / 38.
 static int splitk_of(int64_t M, int64_t N, int64_t K) {
   const int64_t tiles = ((N + kFBN - 1) / kFBN) * ((M + kFBM - 1) / kFBM);
   return tiled(M, N, K) && K >= 96 * kFBK && compute_units() / tiles == 3 ? 3 : 1;
@@ -1477,15 +1480,18 @@ static size_t splitk_bytes(int64_t M, int64_t N, int64_t K) {
 enum class Tile { k64x32, k64x64, k128x64, k128x128, k128x128Pair, k256x128, k256x256 };
 
 // The tile for an [M, N] output (K % 64 == 0). While one of the smaller tiles gives at most one tile
-// per compute unit, the smallest such: a tile's time hardly depends on how many others run (K =
-// 4096, us: 8.5 / 9 / 10.5 / 15 / 28 / 48 for 64x32 / 64x64 / 128x64 / 128x128 / 256x128 / 256x256),
-// so a small output takes the smallest that fits in one round ([16, 1024] at K = 4096 28 -> 8.2 us,
-// [2048, 1024] 30 -> 13.4 us, [1024, 3072] at K = 1024 11.0 -> 8.0 us). Up to two 128 x 128 tiles
-// per unit and K >= 2048, two workgroups share a unit ([4096, 1280] at K = 3392: 32 -> 29 us, the
-// same at K = 1024). Beyond that the rounds of the persistent grid decide between the two large
-// tiles, a round of 256 x 128 tiles taking 0.55 of one of 256 x 256 ([4096, 3392] at K = 1280:
-// 29.0 -> 26.0 us on 224 wide tiles; [8192, 1280] at K = 3392, 160 wide tiles: 62 -> 52 us).
-// Figures with operands that alternate among buffers larger than the L2s.
+// per compute unit, the smallest such: a tile's time hardly depends on how many others run (N = 1024, K
+// = 4096, us, 28 to 31 on 256 x 128 tiles: 16 rows 8.1 and 512 rows 8.9 on 64 x 32, 1024 rows 10.4 on
+// 64 x 64, 2048 rows 13.4 on 128 x 64, 4096 rows 20 on 128 x 128; [1024, 3072] at K = 1024 11.3 ->
+// 8.1). Up to two 128 x 128 tiles per unit and K >= 2048, two workgroups share a unit ([4096, 1280] at
+// K = 3392: 32 -> 27.5 us, the same at K = 1024): the better choice with x8 as its quantiser leaves it,
+// in the cache ([8192, 1024] at K = 4096 36.5 -> 35.3 us); where both operands come from HBM, one
+// stage in flight a workgroup is little for a tall output, and 256 x 128 tiles are faster for more than
+// 480 tiles at N = 1024, K >= 3392 (that shape 38 against 36 us) and for 384 or more at N = 512 (up to
+// 11 %). Beyond two per unit the rounds of the persistent grid decide between the two large tiles, a
+// round of 256 x 128 tiles taking 0.55 of one of 256 x 256 ([4096, 3392] at K = 1280: 27.0 -> 24.4 us
+// on 224 wide tiles; [8192, 1280] at K = 3392, 160 wide tiles: 67 -> 56 us).
+// Figures, unless said otherwise, with up to six sets of operands in turn, more than the L2s hold.
 static Tile tile_of(int64_t M, int64_t N, int64_t K, bool narrow_ok) {
   const int64_t cus = compute_units();
   auto count = [M, N](int64_t bn, int64_t bm) { return ((N + bn - 1) / bn) * ((M + bm - 1) / bm); };
@@ -1622,11 +1628,14 @@ static int scaled_mm(const uint8_t* x8, int64_t M, int64_t K, const uint8_t* w8,
 }
 
 // The W8A16 product's tile: while 64 x 64 or 128 x 64 (n x m) give at most one tile per compute unit,
-// the first of them ([200, 3840] at K = 1280 30.6 -> 8.6 us, [512, 1024] at K = 4096 83 -> 20, [2048,
-// 1024] at K = 4096 85 -> 25); beyond that 128 x 128 tiles, two workgroups a unit, or 256 x 256, by
+// the first of them ([200, 3840] at K = 1280 30.6 -> 8.8 us, [512, 1024] at K = 4096 83 -> 20, [2048,
+// 1024] at K = 4096 84 -> 30); beyond that 128 x 128 tiles, two workgroups a unit, or 256 x 256, by
 // the rounds: in units of a 256 x 256 round a full one of the pairs takes 0.64, a last one of at most
-// a tile per unit 0.39 ([4096, 1024] at K = 1024 26 -> 13 us, [8192, 3072] 63 -> 55; [8192, 4096] stays
-// on 256 x 256 tiles, 67 against 74 us). Results do not depend on the tile.
+// a tile per unit 0.39 ([4096, 1024] at K = 1024 26.5 -> 13.7 us, [8192, 3072] 68 -> 64; [8192, 4096]
+// stays on 256 x 256 tiles, 67 against 74 us). Where the two come out close, at four rounds of pairs
+// and a short one against three, the operands' place decides: [10058, 3392] at K = 1280 112 us on pairs
+// against 106 from HBM, 109 against 112 in the cache, [8780, 3840] 104 either way and 99 against 109.
+// Results do not depend on the tile.
 static TileKernel w8a16_tile_kernel(int64_t M, int64_t N) {
   const int64_t cus = compute_units();
   auto count = [M, N](int64_t bn, int64_t bm) { return ((N + bn - 1) / bn) * ((M + bm - 1) / bm); };

@@ -423,7 +423,8 @@ int flw_gelu_quant_rows_e4m3(const void* x, int64_t rows, int64_t cols, int64_t 
  *   backward (the reference's _swa_fwd, :84-160).
  * flw_swa_bf16_bwd: dq, dk, dv from dout and the forward's out / lse (the reference's
  *   _swa_bwd_preprocess, _swa_bwd_dkdv and _swa_bwd_dq, :163-305); the workspace holds
- *   Delta = rowsum(dout * out). */
+ *   Delta = rowsum(dout * out). dq, dk and dv overlap no other argument (they are written while the
+ *   inputs are still read). */
 int flw_swa_bf16_fwd(const void* q, const void* k, const void* v, int64_t B, int64_t H, int64_t T,
                      int64_t D, int64_t window, void* out, float* lse, void* stream);
 /* flw_swa_bf16_fwd writing O in out_layout: FLW_LAYOUT_BHTD (as flw_swa_bf16_fwd) or
