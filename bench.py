@@ -1016,7 +1016,7 @@ def bench_linear_train(cfg, steps, warmup):
     mws = torch.empty(max(256, lib.flw_fp8_scaled_mm_workspace_bytes(M, N, K), lib.flw_fp8_scaled_mm_workspace_bytes(M, K, N),
                           lib.flw_fp8_scaled_mm_workspace_bytes(N, K, Mp)), dtype=torch.uint8, device="cuda")
 
-    def mm(a8, sa, b8, sb, out, m, n, k):     # split over K into mws when [m, n] has few tiles
+    def mm(a8, sa, b8, sb, out, m, n, k):     # split over K into mws where the entry point does
         C(lib.flw_fp8_scaled_mm_ws(a8.data_ptr(), m, k, b8.data_ptr(), n, sa.data_ptr(), sa.numel(),
                                    sb.data_ptr(), sb.numel(), out.data_ptr(), n, mws.data_ptr(), mws.numel(),
                                    stream), "mm")

@@ -361,8 +361,8 @@ class Fp8DecoderBlock(nn.Module):
             # The quantisation point of qkv_heads (base.py:630-637) in the QKV GEMM's epilogue: the q
             # and k heads are QK-normed and rotated before they are stored, and the per-head maxima
             # of q', k', v come with them, so the attention's quantiser runs only its quantise pass
-            # (K / V codes; Q is quantised on load by the attention kernel). The 256 x 256 GEMM
-            # (K % 128 == 0, operands < 2^32 bytes) carries this epilogue; other shapes take the
+            # (K / V codes; Q is quantised on load by the attention kernel). The tiled GEMM kernels
+            # (K % 128 == 0, operands < 2^32 bytes) carry this epilogue; other shapes take the
             # quantiser pair below.
             w8, ws = qkv_l.weight_codes()
             qkv, amax = native.qkv_norm_rope_amax(c1, s1, w8, ws, att.head_dim, qk_norm, float(eps), cos, sin, T, stream)

@@ -8,19 +8,18 @@
 // ONE query and the softmax row reductions are lane-local plus one v_permlane32_swap), the online
 // softmax in base 2, P packed to bf16 straight from those registers into the B operand of
 // O^T += V^T P^T. For that the K order of each 16-deep k-step is permuted: lane half h takes the
-// keys {0-3, 8-11} + 4h of the step, exactly the scores it already holds, and the V^T tile in LDS
-// is stored in that order (V is transposed while it is staged). L = m + log(l) is written for the
-// backward.
+// keys {0-3, 8-11} + 4h of the step, exactly the scores it already holds, and V^T is read from the V
+// tile in LDS in that order. L = m + log(l) is written for the backward.
 //
 // Backward (after Delta = rowsum(dO * O)):
 //   dK / dV: one workgroup = 128 keys (4 waves x 32 keys, their K and V fragments in registers),
 //     walking the 64-query tiles that see them. S = Q K^T and dP = dO V^T with queries as MFMA
 //     rows, so a lane holds 16 queries of ONE key; P = exp(S - L), dS = P (dP - Delta) / sqrt(D)
 //     feed dV += P^T dO and dK += dS^T Q directly as A operands (the same k-step permutation over
-//     queries), with dO^T and Q^T staged transposed in LDS.
+//     queries), with dO^T and Q^T read transposed from LDS.
 //   dQ: one workgroup = 128 queries (Q and dO fragments in registers), walking key tiles:
 //     S^T = K Q^T, dP^T = V dO^T (keys as rows, one query per lane), dS^T, then
-//     dQ^T += K^T dS^T with K^T staged transposed in LDS.
+//     dQ^T += K^T dS^T with K^T read transposed from LDS.
 // Rows past T are loaded as zeros and never stored.
 #include <math.h>
 

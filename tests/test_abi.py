@@ -92,7 +92,7 @@ def test_host_only_calls_work_without_a_gpu():
     rc = lib.flw_fp8_linear(16, 8, 80, 80, 16, 16, 16, 16, 1, 16, 16, None, 0, None)   # W8A16
     assert rc == 2 and b"multiple of 64" in lib.flw_last_error()
     assert lib.flw_fp8_scaled_mm_workspace_bytes(8192, 4096, 1024) == 0    # 512 tiles: no split
-    assert lib.flw_fp8_scaled_mm_workspace_bytes(256, 256, 100) == 0       # K % 128: no split
+    assert lib.flw_fp8_scaled_mm_workspace_bytes(256, 256, 100) == 0       # K % 64: no split
     # a workspace only where the GEMM splits: three ranges of the fp32 output, K >= 12288 (256 compute units)
     assert lib.flw_fp8_scaled_mm_workspace_bytes(3840, 1280, 16384) == 3 * 3840 * 1280 * 4
     assert lib.flw_fp8_scaled_mm_workspace_bytes(3392, 1276, 12352) == 3 * 3392 * 1276 * 4
@@ -161,7 +161,7 @@ def test_limits_and_empty_shapes_are_refused_on_the_host():
     assert rc == 3 and b"workspace" in lib.flw_last_error()
     rc = lib.flw_amax_e4m3(P, _lib.BF16, 1, 2, 64, 64, 8192, 4096, 64, 7, P, P, 1 << 20, None)
     assert rc == 1 and b"granularity" in lib.flw_last_error()
-    # the QKV GEMM's group amax exists only in the 256 x 256 kernel: operands past 2^32 bytes
+    # the QKV GEMM's group amax exists only in the tiled kernels: operands past 2^32 bytes
     # (M * K = 2^32 here) are refused instead of returning an unwritten amax
     rc = lib.flw_fp8_scaled_mm_group_amax(P, 1 << 22, 1024, P, 256, P, 1 << 22, P, 256, P, 256, 64, P, None)
     assert rc == 2 and b"group amax" in lib.flw_last_error()

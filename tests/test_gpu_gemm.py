@@ -36,9 +36,9 @@ def codes(shape, seed):
                                    (5120, 3328, 128), (4900, 1280, 320)])
 @pytest.mark.parametrize("sx_per_row,sw_per_col", [(True, True), (False, False), (True, False)])
 def test_scaled_mm_matches_closed_form(M, N, K, sx_per_row, sw_per_col):
-    """The 256-tile kernel against the closed form: small and ragged shapes, and outputs with more
-    256 x 256 tiles than compute units whose last round the 256 x 128 tiles fill better (260 tiles;
-    a ragged 100 with K % 128 == 64)."""
+    """Against the closed form: small and ragged shapes (64 x 32 tiles, or the general kernel where K %
+    64 != 0), and two outputs on 256 x 128 tiles (260 tiles of 256 x 256, more than compute units; a
+    ragged 100 with K % 128 == 64)."""
     from flower_amd import _lib as L
     lb = L.load()
     x8, w8 = codes((M, K), 1), codes((N, K), 2)
@@ -351,8 +351,8 @@ def test_fp8_lm_head_matches_bf16_head(shift):
 @pytest.mark.parametrize("M,N,K", [(512, 1024, 1024), (300, 260, 128), (100, 36, 80), (512, 1024, 320)])
 def test_scaled_mm_residual_epilogue(M, N, K):
     """flw_fp8_scaled_mm_residual: y = bf16(residual + bf16(scaled product)), against the closed
-    form with both roundings; the 256-tile kernel (K % 64 == 0; 320 ends on a 64-deep stage) and
-    the general one."""
+    form with both roundings; the 64 x 32 tiles (K % 64 == 0; 320 ends on a 64-deep stage) and
+    the general kernel."""
     from flower_amd import _lib as L
     from oracle.e4m3 import round_bf16
     lb = L.load()
